@@ -72,6 +72,38 @@ def _params_dict(flat):
     return po.unflatten(np.asarray(flat, np.float64))
 
 
+@pytest.mark.parametrize("groups,group", [(1, 2), (3, 11), (1, 64), (5, 103), (2, 257), (130, 64), (65, 253)])
+def test_gradients_of_ragged_batches(groups, group):
+    """Row counts around the tile (64 rows), the k step (32 rows), the split
+    (256 rows) and the column chunk (512 chunks of 32 rows) of the training
+    kernels.  Tolerance: bf16 operands round at 2^-9, so a hidden unit near
+    zero may fall on the other side of its relu; 5e-3 of the gradient's norm
+    as in the check against the oracle above."""
+    rows = groups * group
+    rng = np.random.default_rng(rows)
+    proposer = prop.Proposer(0, seed=3)
+    try:
+        x = torch.from_numpy(rng.standard_normal((rows, 128)).astype(np.float32)).to("cuda:0").to(torch.bfloat16)
+        t = rng.random((groups, group)).astype(np.float32)
+        t /= t.sum(axis=1, keepdims=True)
+        print(f"[proposer] gradients of {groups} x {group} rows", flush=True)
+        grads, losses = proposer.gradients(x, torch.from_numpy(t.ravel()).to("cuda:0"), group)
+        torch.cuda.synchronize()
+        pd = _params_dict(proposer.get_params())
+        cache = po.forward(pd, x.float().cpu().numpy(), emulate_bf16=True)
+        loss, ds = po.listwise_loss(cache["s"], t.ravel(), group)
+        np.testing.assert_allclose(losses.cpu().numpy().mean(), loss, rtol=1e-4)
+        want = po.backward(pd, cache, ds, emulate_bf16=True)
+        got = po.unflatten(grads.cpu().numpy().astype(np.float64))
+        for name, _ in po.SHAPES[:-1]:
+            err = np.linalg.norm(got[name] - want[name]) / max(np.linalg.norm(want[name]), 1e-30)
+            assert err <= 5e-3, f"{name}: {err:.2e}"
+        # db3 sums softmax - targets, 0 per group up to rounding.
+        assert abs(float(got["b3"][0])) <= 1e-6
+    finally:
+        proposer.close()
+
+
 def test_features_scores_and_gradients_match_the_oracle():
     params = parse_stage_parameters(BASIC, ARGS)
     ctx = vnlbhip.Context(0)

@@ -7,6 +7,7 @@
 // Matrix products run on the matrix cores (v_mfma_f32_16x16x32_bf16: bf16
 // operands, fp32 accumulation) in one generic tiled kernel; the fp32 master
 // weights take Adam steps and are copied to bf16 for the products.
+#include <algorithm>
 #include <cfloat>
 
 #include "kernels.h"
@@ -83,21 +84,73 @@ __global__ void features_kernel(const float* __restrict__ clip, int width, int h
     }
 }
 
-template <class T> __device__ inline float load_as_float(const T* p) { return static_cast<float>(*p); }
+// Eight consecutive operand elements as bf16 (fp32 ones rounded to nearest
+// even), from a 16-byte aligned address.
+__device__ inline prop_bf16x8 load8(const __bf16* p) { return *reinterpret_cast<const prop_bf16x8*>(p); }
+__device__ inline prop_bf16x8 load8(const float* p) {
+    const prop_floatx4 lo = *reinterpret_cast<const prop_floatx4*>(p);
+    const prop_floatx4 hi = *reinterpret_cast<const prop_floatx4*>(p + 4);
+    prop_bf16x8 out;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        out[i] = static_cast<__bf16>(lo[i]);
+        out[4 + i] = static_cast<__bf16>(hi[i]);
+    }
+    return out;
+}
 
-// C[m][n] = sum_k A(m, k) B(k, n) with A(m, k) = a[m * a_rs + k * a_cs] and
-// B(k, n) = b[k * b_rs + n * b_cs], operands rounded to bf16 when staged.
-// 64 x 64 output tiles, four waves of 32 x 32.  Epilogue: + bias[n] when
-// given; fp32 result to c32 (ldc) and/or relu(result) as bf16 to c16.
-template <class TA, class TB>
-__global__ __launch_bounds__(256) void gemm_kernel(int M, int N, int K, const TA* __restrict__ a, long long a_rs,
-                                                   long long a_cs, const TB* __restrict__ b, long long b_rs,
-                                                   long long b_cs, const float* __restrict__ bias,
+// This thread's eight elements of a staged 64 x 32 operand tile (rows
+// i0 .. i0 + 63, k0 .. k0 + 31).  kAlongK: the operand is [i][k] with k
+// contiguous (extent k_end a multiple of 32, rows past `extent` are zero);
+// else it is [k][i] with i contiguous (extent a multiple of 64, k past k_end
+// is zero).
+template <bool kAlongK, class T>
+__device__ inline prop_bf16x8 tile_load(const T* __restrict__ p, int ld, int i0, int extent, int k0, int k_end) {
+    const int i = kAlongK ? i0 + (threadIdx.x >> 2) : i0 + (threadIdx.x & 7) * 8;
+    const int k = kAlongK ? k0 + (threadIdx.x & 3) * 8 : k0 + (threadIdx.x >> 3);
+    prop_bf16x8 zero{};
+    if (kAlongK) {
+        return i < extent ? load8(p + static_cast<size_t>(i) * ld + k) : zero;
+    }
+    return k < k_end ? load8(p + static_cast<size_t>(k) * ld + i) : zero;
+}
+
+template <bool kAlongK>
+__device__ inline void tile_store(__bf16* __restrict__ s, const prop_bf16x8& v) {
+    if constexpr (kAlongK) {
+        *reinterpret_cast<prop_bf16x8*>(s + (threadIdx.x >> 2) * kGemmPitch + (threadIdx.x & 3) * 8) = v;
+    } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            s[((threadIdx.x & 7) * 8 + j) * kGemmPitch + (threadIdx.x >> 3)] = v[j];
+        }
+    }
+}
+
+// C[m][n] = sum_k A(m, k) B(k, n), operands rounded to bf16 when staged;
+// kAK: A is [m][k], else [k][m]; kBK: B is [n][k], else [k][n] (leading
+// dimensions lda, ldb; see tile_load for the extents).  64 x 64 output
+// tiles, four waves of 32 x 32; the next k step's operands are loaded (16
+// bytes per load) while this one is on the matrix cores.  Epilogue: +
+// bias[n] when given, zero where mask[m][n] <= 0 when given; fp32 result to
+// c32 (ldc) and/or relu(result) as bf16 to c16.
+//
+// Split K: workgroup z sums k in [z per_split, (z + 1) per_split) into
+// c32 + z M ldc.  The weight gradients contract over the batch's rows (8192
+// for 64 anchors) into 256 x 256 and 256 x 128 results, 16 and 8 tiles for
+// 256 compute units: unsplit, each of them took 1.3 ms of latency-bound
+// steps; with 32 splits and the step pipeline the two average 14 us.
+template <bool kAK, bool kBK, class TA, class TB>
+__global__ __launch_bounds__(256) void gemm_kernel(int M, int N, int K, int per_split, const TA* __restrict__ a,
+                                                   int lda, const TB* __restrict__ b, int ldb,
+                                                   const float* __restrict__ bias, const float* __restrict__ mask,
                                                    float* __restrict__ c32, __bf16* __restrict__ c16, int ldc) {
     __shared__ __attribute__((aligned(16))) __bf16 s_a[kGemmTile * kGemmPitch];
     __shared__ __attribute__((aligned(16))) __bf16 s_b[kGemmTile * kGemmPitch];
     const int m0 = blockIdx.y * kGemmTile;
     const int n0 = blockIdx.x * kGemmTile;
+    const int k_begin = blockIdx.z * per_split;
+    const int k_end = min(K, k_begin + per_split);
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int col = lane & 15;
@@ -112,34 +165,20 @@ __global__ __launch_bounds__(256) void gemm_kernel(int M, int N, int K, const TA
             acc[i][j] = prop_floatx4{0.0F, 0.0F, 0.0F, 0.0F};
         }
     }
-    // Staging order: k fastest when the operand is k-contiguous, else the
-    // row index fastest.
-    const bool a_k_fast = a_cs == 1;
-    const bool b_k_fast = b_rs == 1;
-    for (int k0 = 0; k0 < K; k0 += kGemmK) {
-        for (int e = threadIdx.x; e < kGemmTile * kGemmK; e += blockDim.x) {
-            const int i = a_k_fast ? e / kGemmK : e % kGemmTile;
-            const int k = a_k_fast ? e % kGemmK : e / kGemmTile;
-            const int m = m0 + i;
-            const int kk = k0 + k;
-            float v = 0.0F;
-            if (m < M && kk < K) {
-                v = load_as_float(a + m * a_rs + kk * a_cs);
-            }
-            s_a[i * kGemmPitch + k] = static_cast<__bf16>(v);
-        }
-        for (int e = threadIdx.x; e < kGemmTile * kGemmK; e += blockDim.x) {
-            const int j = b_k_fast ? e / kGemmK : e % kGemmTile;
-            const int k = b_k_fast ? e % kGemmK : e / kGemmTile;
-            const int n = n0 + j;
-            const int kk = k0 + k;
-            float v = 0.0F;
-            if (n < N && kk < K) {
-                v = load_as_float(b + kk * b_rs + n * b_cs);
-            }
-            s_b[j * kGemmPitch + k] = static_cast<__bf16>(v);
-        }
+    prop_bf16x8 ra{};
+    prop_bf16x8 rb{};
+    if (k_begin < k_end) {
+        ra = tile_load<kAK>(a, lda, m0, M, k_begin, k_end);
+        rb = tile_load<kBK>(b, ldb, n0, N, k_begin, k_end);
+    }
+    for (int k0 = k_begin; k0 < k_end; k0 += kGemmK) {
+        tile_store<kAK>(s_a, ra);
+        tile_store<kBK>(s_b, rb);
         __syncthreads();
+        if (k0 + kGemmK < k_end) {
+            ra = tile_load<kAK>(a, lda, m0, M, k0 + kGemmK, k_end);
+            rb = tile_load<kBK>(b, ldb, n0, N, k0 + kGemmK, k_end);
+        }
         prop_bf16x8 av[2];
         prop_bf16x8 bv[2];
 #pragma unroll
@@ -156,6 +195,7 @@ __global__ __launch_bounds__(256) void gemm_kernel(int M, int N, int K, const TA
         }
         __syncthreads();
     }
+    float* __restrict__ out32 = c32 + static_cast<size_t>(blockIdx.z) * M * ldc;
     // acc[i][j][v] = C[wm + 16 i + 4 kb + v][wn + 16 j + col]
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
@@ -170,12 +210,14 @@ __global__ __launch_bounds__(256) void gemm_kernel(int M, int N, int K, const TA
             for (int v = 0; v < 4; ++v) {
                 const int m = m0 + wm + 16 * i + 4 * kb + v;
                 if (m < M) {
-                    const float z = acc[i][j][v] + add;
-                    if (c32 != nullptr) {
-                        c32[static_cast<size_t>(m) * ldc + n] = z;
+                    const size_t at = static_cast<size_t>(m) * ldc + n;
+                    float z = acc[i][j][v] + add;
+                    if (mask != nullptr && !(mask[at] > 0.0F)) {
+                        z = 0.0F;
                     }
+                    out32[at] = z;
                     if (c16 != nullptr) {
-                        c16[static_cast<size_t>(m) * ldc + n] = static_cast<__bf16>(z > 0.0F ? z : 0.0F);
+                        c16[at] = static_cast<__bf16>(z > 0.0F ? z : 0.0F);
                     }
                 }
             }
@@ -248,79 +290,123 @@ __global__ void loss_kernel(const float* __restrict__ s, const float* __restrict
     }
 }
 
-// dz2[m][n] = ds[m] w3[n] (z2 > 0)
-__global__ void output_grad_kernel(const float* __restrict__ z2, const float* __restrict__ ds,
-                                   const float* __restrict__ params, int rows, float* __restrict__ dz2) {
-    const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= static_cast<size_t>(rows) * kPropHidden) {
-        return;
-    }
-    const int n = static_cast<int>(i % kPropHidden);
-    const size_t m = i / kPropHidden;
-    dz2[i] = z2[i] > 0.0F ? ds[m] * params[kOffW3 + n] : 0.0F;
+// Column sums over the batch's rows go through partial sums of row chunks, in
+// row order within a chunk; reduce_kernel adds the chunks.
+constexpr int kColChunkRows = 32;
+constexpr int kColMaxChunks = 512;
+
+__host__ __device__ inline int column_chunk_rows(int rows) {
+    const int per = (rows + kColMaxChunks - 1) / kColMaxChunks;
+    return per > kColChunkRows ? per : kColChunkRows;
 }
 
-// dz[m][n] *= (z[m][n] > 0)
-__global__ void relu_mask_kernel(const float* __restrict__ z, float* __restrict__ dz, size_t count) {
-    const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < count && !(z[i] > 0.0F)) {
-        dz[i] = 0.0F;
+// Output layer's backward: dz2[m][n] = ds[m] w3[n] (z2 > 0), and the chunk's
+// partial sums of dw3[n] = sum relu(z2) ds and db2[n] = sum dz2 (thread n,
+// one workgroup per row chunk).
+__global__ __launch_bounds__(kPropHidden) void output_grad_kernel(const float* __restrict__ z2,
+                                                                  const float* __restrict__ ds,
+                                                                  const float* __restrict__ params, int rows,
+                                                                  float* __restrict__ dz2,
+                                                                  float* __restrict__ part_w3,
+                                                                  float* __restrict__ part_b2) {
+    const int n = threadIdx.x;
+    const int per = column_chunk_rows(rows);
+    const int lo = blockIdx.x * per;
+    const int hi = min(rows, lo + per);
+    const float w3 = params[kOffW3 + n];
+    float sum_w3 = 0.0F;
+    float sum_b2 = 0.0F;
+#pragma unroll 8
+    for (int m = lo; m < hi; ++m) {
+        const float z = z2[static_cast<size_t>(m) * kPropHidden + n];
+        const float g = ds[m];
+        const float d = z > 0.0F ? g * w3 : 0.0F;
+        sum_w3 = sum_w3 + (z > 0.0F ? z : 0.0F) * g;
+        sum_b2 = sum_b2 + d;
+        dz2[static_cast<size_t>(m) * kPropHidden + n] = d;
     }
+    part_w3[static_cast<size_t>(blockIdx.x) * kPropHidden + n] = sum_w3;
+    part_b2[static_cast<size_t>(blockIdx.x) * kPropHidden + n] = sum_b2;
 }
 
-constexpr int kColChunks = 64;
-
-// Column sums in two deterministic passes: part[chunk][n] = sum over the
-// chunk's rows (in order) of f(a[m][n]) * (w ? w[m] : 1), f = relu when
-// relu_a; then out[n] = sum over chunks in order.
-__global__ void column_partial_kernel(const float* __restrict__ a, int rows, int cols, const float* __restrict__ w,
-                                      int relu_a, float* __restrict__ part) {
-    const int n = blockIdx.x * blockDim.x + threadIdx.x;
-    const int chunk = blockIdx.y;
-    if (n >= cols) {
-        return;
-    }
-    const int per = (rows + kColChunks - 1) / kColChunks;
-    const int lo = chunk * per;
+// The chunk's partial sums of db1[n] = sum dz1.
+__global__ __launch_bounds__(kPropHidden) void column_partial_kernel(const float* __restrict__ a, int rows,
+                                                                     float* __restrict__ part) {
+    const int n = threadIdx.x;
+    const int per = column_chunk_rows(rows);
+    const int lo = blockIdx.x * per;
     const int hi = min(rows, lo + per);
     float sum = 0.0F;
+#pragma unroll 8
     for (int m = lo; m < hi; ++m) {
-        float v = a[static_cast<size_t>(m) * cols + n];
-        if (relu_a != 0) {
-            v = v > 0.0F ? v : 0.0F;
-        }
-        sum = sum + (w != nullptr ? v * w[m] : v);
+        sum = sum + a[static_cast<size_t>(m) * kPropHidden + n];
     }
-    part[static_cast<size_t>(chunk) * cols + n] = sum;
+    part[static_cast<size_t>(blockIdx.x) * kPropHidden + n] = sum;
 }
 
-__global__ void column_total_kernel(const float* __restrict__ part, int cols, float* __restrict__ out) {
-    const int n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= cols) {
+// Adds the partial results of a batch into the flat gradient, every sum in a
+// fixed order: the splits of dW2 and dW1 (one element per thread), the row
+// chunks of dw3, db2 and db1 (16 columns x 16 chunk runs per workgroup) and
+// db3 = sum ds (the last workgroup).
+constexpr int kReduceWeightBlocks = kPropHidden * (kPropHidden + kPropIn) / 256;
+constexpr int kReduceColumnBlocks = 3 * kPropHidden / 16;
+__global__ __launch_bounds__(256) void reduce_kernel(const float* __restrict__ part_weights, int splits,
+                                                     const float* __restrict__ part_columns, int chunks,
+                                                     const float* __restrict__ ds, int rows,
+                                                     float* __restrict__ grads) {
+    __shared__ float s_part[256];
+    const int block = blockIdx.x;
+    if (block < kReduceWeightBlocks) {
+        int e = block * 256 + threadIdx.x;
+        const bool second = e < kPropHidden * kPropHidden;
+        const int size = kPropHidden * (second ? kPropHidden : kPropIn);
+        const float* p = part_weights;
+        if (!second) {
+            e -= kPropHidden * kPropHidden;
+            p += static_cast<size_t>(splits) * kPropHidden * kPropHidden;
+        }
+        float sum = 0.0F;
+#pragma unroll 8
+        for (int z = 0; z < splits; ++z) {
+            sum = sum + p[static_cast<size_t>(z) * size + e];
+        }
+        grads[(second ? kOffW2 : kOffW1) + e] = sum;
         return;
     }
     float sum = 0.0F;
-    for (int c = 0; c < kColChunks; ++c) {
-        sum = sum + part[static_cast<size_t>(c) * cols + n];
+    if (block < kReduceWeightBlocks + kReduceColumnBlocks) {
+        const int column = (block - kReduceWeightBlocks) * 16 + (threadIdx.x & 15);
+        const int which = column / kPropHidden;
+        const int n = column % kPropHidden;
+        const float* p = part_columns + static_cast<size_t>(which) * chunks * kPropHidden + n;
+#pragma unroll 4
+        for (int c = threadIdx.x >> 4; c < chunks; c += 16) {
+            sum = sum + p[static_cast<size_t>(c) * kPropHidden];
+        }
+        s_part[threadIdx.x] = sum;
+        __syncthreads();
+        if (threadIdx.x < 16) {
+            float total = 0.0F;
+            for (int g = 0; g < 16; ++g) {
+                total = total + s_part[16 * g + threadIdx.x];
+            }
+            grads[(which == 0 ? kOffW3 : (which == 1 ? kOffB2 : kOffB1)) + n] = total;
+        }
+        return;
     }
-    out[n] = sum;
-}
-
-// db3 = sum ds (one block, fixed order).
-__global__ void sum_kernel(const float* __restrict__ v, int count, float* __restrict__ out) {
-    __shared__ float s_part[256];
-    float sum = 0.0F;
-    for (int i = threadIdx.x; i < count; i += blockDim.x) {
-        sum = sum + v[i];
+    for (int i = threadIdx.x; i < rows; i += 256) {
+        sum = sum + ds[i];
     }
     s_part[threadIdx.x] = sum;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        float total = 0.0F;
-        for (int i = 0; i < static_cast<int>(blockDim.x); ++i) {
-            total = total + s_part[i];
+    for (int width = 128; width >= 1; width >>= 1) {
+        if (static_cast<int>(threadIdx.x) < width) {
+            s_part[threadIdx.x] = s_part[threadIdx.x] + s_part[threadIdx.x + width];
         }
-        out[0] = total;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        grads[kOffB3] = s_part[0];
     }
 }
 
@@ -442,21 +528,29 @@ unsigned blocks_for(size_t count, int threads) {
     return static_cast<unsigned>((count + threads - 1) / threads);
 }
 
-template <class TA, class TB>
-hipError_t gemm(int M, int N, int K, const TA* a, long long a_rs, long long a_cs, const TB* b, long long b_rs,
-                long long b_cs, const float* bias, float* c32, __bf16* c16, int ldc, hipStream_t stream) {
-    const dim3 grid(static_cast<unsigned>((N + kGemmTile - 1) / kGemmTile),
-                    static_cast<unsigned>((M + kGemmTile - 1) / kGemmTile));
-    hipLaunchKernelGGL((gemm_kernel<TA, TB>), grid, dim3(256), 0, stream, M, N, K, a, a_rs, a_cs, b, b_rs, b_cs,
-                       bias, c32, c16, ldc);
-    return hipGetLastError();
+// Splits of a contraction over `rows`: at least 256 rows (8 k steps) each,
+// at most 32 (512 workgroups for the 256 x 256 result, two per compute
+// unit; more only adds partial results to sum).
+constexpr int kMaxSplits = 32;
+int weight_splits(int rows) {
+    return std::clamp(rows / 256, 1, kMaxSplits);
 }
 
-hipError_t column_sums(const float* a, int rows, int cols, const float* w, bool relu_a, float* part, float* out,
-                       hipStream_t stream) {
-    hipLaunchKernelGGL(column_partial_kernel, dim3(blocks_for(cols, 64), kColChunks), dim3(64), 0, stream, a, rows,
-                       cols, w, relu_a ? 1 : 0, part);
-    hipLaunchKernelGGL(column_total_kernel, dim3(blocks_for(cols, 64)), dim3(64), 0, stream, part, cols, out);
+template <bool kAK, bool kBK, class TA, class TB>
+hipError_t gemm(int M, int N, int K, int splits, const TA* a, int lda, const TB* b, int ldb, const float* bias,
+                const float* mask, float* c32, __bf16* c16, int ldc, hipStream_t stream) {
+    if ((kAK || kBK) && K % kGemmK != 0) {
+        return hipErrorInvalidValue;
+    }
+    if ((!kAK && M % kGemmTile != 0) || (!kBK && N % kGemmTile != 0)) {
+        return hipErrorInvalidValue;
+    }
+    const int steps = (K + kGemmK - 1) / kGemmK;
+    const int per_split = (steps + splits - 1) / splits * kGemmK;
+    const dim3 grid(static_cast<unsigned>((N + kGemmTile - 1) / kGemmTile),
+                    static_cast<unsigned>((M + kGemmTile - 1) / kGemmTile), static_cast<unsigned>(splits));
+    hipLaunchKernelGGL((gemm_kernel<kAK, kBK, TA, TB>), grid, dim3(256), 0, stream, M, N, K, per_split, a, lda, b,
+                       ldb, bias, mask, c32, c16, ldc);
     return hipGetLastError();
 }
 
@@ -464,9 +558,10 @@ hipError_t column_sums(const float* a, int rows, int cols, const float* w, bool 
 
 size_t proposer_workspace_floats(int rows) {
     // z1, z2, dz2, dz1 (fp32 [rows][256]); h1 (bf16 [rows][256], as floats);
-    // s, ds; column partials.
+    // s, ds; column partials; split partials of dW2 and dW1.
     return static_cast<size_t>(rows) * kPropHidden * 4 + static_cast<size_t>(rows) * kPropHidden / 2 +
-           static_cast<size_t>(rows) * 2 + static_cast<size_t>(kColChunks) * kPropHidden + 64;
+           static_cast<size_t>(rows) * 2 + static_cast<size_t>(3) * kColMaxChunks * kPropHidden +
+           static_cast<size_t>(weight_splits(rows)) * kPropHidden * (kPropHidden + kPropIn) + 64;
 }
 
 hipError_t launch_proposer_init(float* params, uint64_t seed, hipStream_t stream) {
@@ -521,8 +616,8 @@ hipError_t launch_proposer_calibrate(const float* params, const __bf16* w1, cons
     hipLaunchKernelGGL(quantize_rows_kernel, dim3(kPropHidden), dim3(256), 0, stream, params + kOffW1, kPropIn,
                        scales + kPropScaleX, 0, scales, kPropScaleW1, w1_fp8);
     // Hidden activations of the sample with the bf16 weights.
-    hipError_t e = gemm(rows, kPropHidden, kPropIn, x, kPropIn, 1, w1, 1, kPropIn, params + kOffB1, workspace,
-                        static_cast<__bf16*>(nullptr), kPropHidden, stream);
+    hipError_t e = gemm<true, true>(rows, kPropHidden, kPropIn, 1, x, kPropIn, w1, kPropIn, params + kOffB1,
+                                    nullptr, workspace, nullptr, kPropHidden, stream);
     if (e != hipSuccess) {
         return e;
     }
@@ -546,49 +641,49 @@ hipError_t launch_proposer_gradients(const float* params, const __bf16* w1, cons
     __bf16* h1 = reinterpret_cast<__bf16*>(dz1 + wide);
     float* s = dz1 + wide + wide / 2;
     float* ds = s + rows;
-    float* part = ds + rows;
+    const int chunk_rows = column_chunk_rows(rows);
+    const int chunks = (rows + chunk_rows - 1) / chunk_rows;
+    float* part_columns = ds + rows;  // dw3, db2, db1: [chunks][256] each
+    float* part_weights = part_columns + static_cast<size_t>(3) * kColMaxChunks * kPropHidden;
+    const int splits = weight_splits(rows);
+    float* part_w1 = part_weights + static_cast<size_t>(splits) * kPropHidden * kPropHidden;
+    const size_t columns = static_cast<size_t>(chunks) * kPropHidden;
     const int groups = rows / group;
     hipError_t e;
     // Forward.
-    if ((e = gemm(rows, kPropHidden, kPropIn, x, kPropIn, 1, w1, 1, kPropIn, params + kOffB1, z1, h1,
-                  kPropHidden, stream)) != hipSuccess) {
+    if ((e = gemm<true, true>(rows, kPropHidden, kPropIn, 1, x, kPropIn, w1, kPropIn, params + kOffB1, nullptr, z1,
+                              h1, kPropHidden, stream)) != hipSuccess) {
         return e;
     }
-    if ((e = gemm(rows, kPropHidden, kPropHidden, h1, kPropHidden, 1, w2, 1, kPropHidden, params + kOffB2, z2,
-                  static_cast<__bf16*>(nullptr), kPropHidden, stream)) != hipSuccess) {
+    if ((e = gemm<true, true>(rows, kPropHidden, kPropHidden, 1, h1, kPropHidden, w2, kPropHidden, params + kOffB2,
+                              nullptr, z2, nullptr, kPropHidden, stream)) != hipSuccess) {
         return e;
     }
     hipLaunchKernelGGL(output_kernel, dim3(blocks_for(rows, 4)), dim3(256), 0, stream, z2, params, rows, s);
     hipLaunchKernelGGL(loss_kernel, dim3(blocks_for(groups, 4)), dim3(256), 0, stream, s, targets, groups, group,
                        ds, loss_groups);
-    // Output layer.
-    if ((e = column_sums(z2, rows, kPropHidden, ds, true, part, grads + kOffW3, stream)) != hipSuccess) {
+    // Output layer: dz2 and the partial sums of dw3 and db2.
+    hipLaunchKernelGGL(output_grad_kernel, dim3(static_cast<unsigned>(chunks)), dim3(kPropHidden), 0, stream, z2, ds,
+                       params, rows, dz2, part_columns, part_columns + columns);
+    // Layer 2: dW2 = dz2^T h1, dz1 = (dz2 W2) where z1 > 0.
+    if ((e = gemm<false, false>(kPropHidden, kPropHidden, rows, splits, dz2, kPropHidden, h1, kPropHidden, nullptr,
+                                nullptr, part_weights, nullptr, kPropHidden, stream)) != hipSuccess) {
         return e;
     }
-    hipLaunchKernelGGL(sum_kernel, dim3(1), dim3(256), 0, stream, ds, rows, grads + kOffB3);
-    hipLaunchKernelGGL(output_grad_kernel, dim3(blocks_for(wide, 256)), dim3(256), 0, stream, z2, ds, params, rows,
-                       dz2);
-    // Layer 2: dW2 = dz2^T h1, db2 = column sums of dz2, dh1 = dz2 W2.
-    if ((e = column_sums(dz2, rows, kPropHidden, nullptr, false, part, grads + kOffB2, stream)) != hipSuccess) {
+    if ((e = gemm<true, false>(rows, kPropHidden, kPropHidden, 1, dz2, kPropHidden, w2, kPropHidden, nullptr, z1,
+                               dz1, nullptr, kPropHidden, stream)) != hipSuccess) {
         return e;
     }
-    if ((e = gemm(kPropHidden, kPropHidden, rows, dz2, 1, kPropHidden, h1, kPropHidden, 1,
-                  static_cast<const float*>(nullptr), grads + kOffW2, static_cast<__bf16*>(nullptr), kPropHidden,
-                  stream)) != hipSuccess) {
+    // Layer 1: db1 = column sums of dz1, dW1 = dz1^T x.
+    hipLaunchKernelGGL(column_partial_kernel, dim3(static_cast<unsigned>(chunks)), dim3(kPropHidden), 0, stream, dz1,
+                       rows, part_columns + 2 * columns);
+    if ((e = gemm<false, false>(kPropHidden, kPropIn, rows, splits, dz1, kPropHidden, x, kPropIn, nullptr, nullptr,
+                                part_w1, nullptr, kPropIn, stream)) != hipSuccess) {
         return e;
     }
-    if ((e = gemm(rows, kPropHidden, kPropHidden, dz2, kPropHidden, 1, w2, kPropHidden, 1,
-                  static_cast<const float*>(nullptr), dz1, static_cast<__bf16*>(nullptr), kPropHidden,
-                  stream)) != hipSuccess) {
-        return e;
-    }
-    hipLaunchKernelGGL(relu_mask_kernel, dim3(blocks_for(wide, 256)), dim3(256), 0, stream, z1, dz1, wide);
-    // Layer 1: dW1 = dz1^T x, db1 = column sums of dz1.
-    if ((e = column_sums(dz1, rows, kPropHidden, nullptr, false, part, grads + kOffB1, stream)) != hipSuccess) {
-        return e;
-    }
-    return gemm(kPropHidden, kPropIn, rows, dz1, 1, kPropHidden, x, kPropIn, 1, static_cast<const float*>(nullptr),
-                grads + kOffW1, static_cast<__bf16*>(nullptr), kPropIn, stream);
+    hipLaunchKernelGGL(reduce_kernel, dim3(kReduceWeightBlocks + kReduceColumnBlocks + 1), dim3(256), 0, stream,
+                       part_weights, splits, part_columns, chunks, ds, rows, grads);
+    return hipGetLastError();
 }
 
 hipError_t launch_proposer_adam(float* params, const float* grads, float* m, float* v, float lr, int step,
