@@ -13,7 +13,7 @@ import torch
 
 import workloads
 from vnlbhip import synth
-from vnlbhip.params import BASIC, FINAL, StageParameters
+from vnlbhip.params import BASIC, FINAL, StageParameters, parse_stage_parameters
 
 pytestmark = pytest.mark.gpu
 
@@ -69,6 +69,22 @@ def test_match_paste_model_bitwise(gpu, oracle_lib, name):
     basic, _ = oracle_lib.stage(BASIC, bp, noisy, flags=oracle_lib.ACCUM_DOUBLE, threads=4)
     for af in sorted({0, 2, frames - fp.patch_time}):
         _compare_frame(gpu, oracle_lib, FINAL, fp, noisy, basic, af)
+
+
+@pytest.mark.parametrize("patch_size,group_size", [
+    (8, 2), (8, 3), (8, 4), (8, 5), (8, 8), (8, 9), (8, 12), (8, 13), (8, 16), (8, 17), (8, 31), (8, 32), (8, 33),
+    (8, 63), (8, 64), (8, 65), (8, 100), (8, 112), (9, 90), (11, 122), (3, 40), (5, 60)])
+def test_eigen_solver_sizes(gpu, oracle_lib, patch_size, group_size):
+    """Eigen problems at the edges of the solvers' sizes (4, 8, 12, 16, 32, 64
+    and 128 rows), dual (8x8x2 patches) and covariance (121, 81, 25 and 9 samples per
+    patch) ones: eigenvalues bit for bit, weights from the eigenvectors."""
+    noisy, _ = synth.make_clip(40, 36, 4, 1, sigma8=15, seed=90 + group_size, motion="subpixel")
+    args = dict(sigma=15, block_size=patch_size, block_step=6, group_size=group_size, bm_range=6, radius=1, tau=0,
+                patch_time=2 if patch_size == 8 else 1, rank=min(group_size, 20, patch_size * patch_size))
+    bp = parse_stage_parameters(BASIC, args)
+    print(f"[parity] {patch_size}x{patch_size} patches, {group_size} neighbours", flush=True)
+    want = _compare_frame(gpu, oracle_lib, BASIC, bp, noisy, None, 1)
+    assert ((want["group_flags"] & 4) != 0).any()
 
 
 @pytest.mark.parametrize("name", list(workloads.WORKLOADS))

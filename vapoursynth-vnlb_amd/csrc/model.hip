@@ -25,26 +25,268 @@ namespace {
 // max_sweeps sweeps, "converged" also when the off-diagonal is below
 // 8 * threshold; eigenpairs sorted descending (stable) and each vector made
 // unit length with its largest-magnitude entry positive
-// (canonicalize_vector_row :204-233).  Each lane owns one matrix row.
-// kLP = 128 (n up to 128, the dual Grams of up to 128 model rows): one
-// problem per block of two wavefronts; the segment reductions then go
-// through LDS and the rotation loops stop at the problem's n (uniform in the
-// block).
-template <int kLP>  // lanes per problem (power of two >= n)
-__global__ __launch_bounds__(128) void jacobi_kernel(
+// (canonicalize_vector_row :204-233).
+//
+// Both kernels below apply the rotations in the reference's order with its
+// operations, so their results are the reference's bit for bit.  They share
+// one observation: while the rotations (p, p + 1), (p, p + 2), ... of row p
+// run, row r only needs its running entry A[r][p], its entry A[r][q] of the
+// current column and the same two of V; what the symmetric copies of row p
+// hold is read by nobody until the row is finished.
+
+// jacobi_rotate (linalg.cpp:153-202): the rotation of pivot apq between the
+// diagonal entries app and aqq, and the new diagonal.
+struct Rotation {
+    float c;
+    float s;
+    float new_pp;
+    float new_qq;
+};
+
+// Square root and reciprocal of x >= 1, correctly rounded: the hardware's
+// approximation and one Newton step on its residual.  Compared with sqrtf
+// and 1.0F / x for every float in [1, 2^32): no difference (both depend on
+// the mantissa and, for the root, the exponent's parity alone).  Without the
+// general case's scaling and special values they are 4 and 3 dependent
+// instructions instead of 15 and 11.
+__device__ __forceinline__ float sqrt_from_one(float x) {
+    const float y = __builtin_amdgcn_rsqf(x);
+    const float s = x * y;
+    return fmaf(fmaf(-s, s, x), 0.5F * y, s);
+}
+__device__ __forceinline__ float reciprocal_from_one(float x) {
+    const float r = __builtin_amdgcn_rcpf(x);
+    return fmaf(fmaf(-x, r, 1.0F), r, r);
+}
+
+// A rotating pivot is above 64 float epsilons of max |A| and the diagonal at
+// most n max |A| = 128 max |A|, so |tau| is below 2^25 and the two roots and
+// reciprocals stay within the range above.
+__device__ __forceinline__ Rotation rotation_of(float app, float aqq, float apq) {
+    Rotation o;
+    const float tau = (aqq - app) / (2.0F * apq);
+    const float tau_abs = fabsf(tau);
+    const float t_abs = reciprocal_from_one(tau_abs + sqrt_from_one(1.0F + (tau * tau)));
+    const float t = tau < 0.0F ? -t_abs : t_abs;
+    o.c = reciprocal_from_one(sqrt_from_one(1.0F + (t * t)));
+    o.s = t * o.c;
+    const float cc = o.c * o.c;
+    const float ss = o.s * o.s;
+    const float two_cs = 2.0F * (o.c * o.s);
+    o.new_pp = ((cc * app) - (two_cs * apq)) + (ss * aqq);
+    o.new_qq = ((ss * app) + (two_cs * apq)) + (cc * aqq);
+    return o;
+}
+
+__device__ inline void rotate_pair(const Rotation& o, float& left, float& right) {
+    const float l = left;
+    const float r = right;
+    left = (o.c * l) - (o.s * r);
+    right = (o.s * l) + (o.c * r);
+}
+
+// The kRank-th eigenpair from V (rows of `stride` floats in LDS) and the
+// diagonal: the canonical vector of column col, read in row order.
+__device__ inline void write_eigenvector(const float* __restrict__ v, int stride, int n, int col,
+                                         float* __restrict__ out) {
+    float norm_squared = 0.0F;
+    float max_abs = 0.0F;
+    int pivot = 0;
+    for (int i = 0; i < n; ++i) {
+        const float value = v[i * stride + col];
+        const float square = value * value;
+        norm_squared = norm_squared + square;
+        const float value_abs = fabsf(value);
+        if (value_abs > max_abs) {
+            max_abs = value_abs;
+            pivot = i;
+        }
+    }
+    float scale = 1.0F;
+    const bool rescale = norm_squared > FLT_MIN;
+    if (rescale) {
+        scale = 1.0F / sqrtf(norm_squared);
+        if (v[pivot * stride + col] < 0.0F) {
+            scale = -scale;
+        }
+    }
+    for (int i = 0; i < n; ++i) {
+        const float value = v[i * stride + col];
+        out[i] = rescale ? value * scale : value;
+    }
+}
+
+// v of lane kLane of the same four lanes.
+template <int kLane> __device__ inline float quad_lane(float v) {
+    return __builtin_bit_cast(
+        float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), kLane * 0x55, 0xF, 0xF, true));
+}
+
+// A value the compiler has to have in a register here: keeps it from turning
+// a chain of cases over one register array into an indexed array in memory.
+__device__ __forceinline__ float pinned(float v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
+// Problems of at most 4 kSlots (<= 16) rows: four lanes per problem, sixteen
+// problems per wavefront, A and V in registers; lane l holds the rows
+// l, l + 4, ... (slot k is row 4 k + l).  Bound by instruction issue: a
+// rotation's divide, roots and reciprocals (about 50 instructions) cost the
+// wavefront the same whether 4 or 16 problems share it, so four lanes per
+// problem beat sixteen; one lane per problem would need A and V of 16 rows in
+// 392 registers.  Measured against sixteen lanes per problem with A and V in
+// LDS, half a stage each: 188 k problems of 16 rows 4.60 -> 1.67 ms, 83 k of
+// 12 rows 1.24 -> 0.38 ms, 2.6 k of 8 rows 79 -> 46 us (a wavefront's serial
+// chain).
+template <int kSlots, int kP>
+__device__ __forceinline__ void quad_load_row(const float (&a)[kSlots][4 * kSlots], const float (&v)[kSlots][4 * kSlots],
+                                     int p, float (&rp)[kSlots], float (&vp)[kSlots], float& app) {
+    if (p == kP) {
+#pragma unroll
+        for (int k = 0; k < kSlots; ++k) {
+            rp[k] = pinned(a[k][kP]);
+            vp[k] = pinned(v[k][kP]);
+        }
+        app = quad_lane<kP % 4>(pinned(a[kP / 4][kP]));
+    }
+}
+
+// Row p finished: column p and row p of A (entries rp, diagonal app).
+template <int kSlots, int kP, int... kX>
+__device__ __forceinline__ void quad_store_row(float (&a)[kSlots][4 * kSlots], float (&v)[kSlots][4 * kSlots], int l, int p,
+                                      const float (&rp)[kSlots], const float (&vp)[kSlots], float app,
+                                      std::integer_sequence<int, kX...>) {
+    if (p == kP) {
+#pragma unroll
+        for (int k = 0; k < kSlots; ++k) {
+            a[k][kP] = pinned(rp[k]);
+            v[k][kP] = pinned(vp[k]);
+        }
+        // (The lane exchanges run in all lanes of the four, the selects after them.)
+        const bool own = l == kP % 4;
+        const auto take = [&](float& entry, float value) { entry = own ? value : entry; };
+        (take(a[kP / 4][kX], quad_lane<kX % 4>(rp[kX / 4])), ...);
+        a[kP / 4][kP] = own ? app : a[kP / 4][kP];
+    }
+}
+
+// Rotation (p, kQ).  The lane of row kQ takes the new column's entries as
+// its row; row p's entries are junk until quad_store_row.
+template <int kSlots, int kQ, int... kX>
+__device__ __forceinline__ void quad_rotate(float (&a)[kSlots][4 * kSlots], float (&v)[kSlots][4 * kSlots], int l, int p,
+                                   bool active, float threshold, float (&rp)[kSlots], float (&vp)[kSlots],
+                                   float& app, std::integer_sequence<int, kX...>) {
+    if (kQ <= p) {
+        return;  // uniform
+    }
+    const float apq = quad_lane<kQ % 4>(rp[kQ / 4]);
+    if (active && fabsf(apq) > threshold) {
+        const float aqq = quad_lane<kQ % 4>(a[kQ / 4][kQ]);
+        const Rotation o = rotation_of(app, aqq, apq);
+        app = o.new_pp;
+#pragma unroll
+        for (int k = 0; k < kSlots; ++k) {
+            rotate_pair(o, rp[k], a[k][kQ]);
+            rotate_pair(o, vp[k], v[k][kQ]);
+        }
+        const bool own = l == kQ % 4;
+        rp[kQ / 4] = own ? 0.0F : rp[kQ / 4];
+        const auto take = [&](float& entry, float value) { entry = own ? value : entry; };
+        (take(a[kQ / 4][kX], quad_lane<kX % 4>(a[kX / 4][kQ])), ...);
+        a[kQ / 4][kQ] = own ? o.new_qq : a[kQ / 4][kQ];
+    }
+    // One rotation at a time (bounded register use).
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+template <int kSlots, int... kI>
+__device__ __forceinline__ void quad_sweep(float (&a)[kSlots][4 * kSlots], float (&v)[kSlots][4 * kSlots], int l, bool active,
+                                  float threshold, std::integer_sequence<int, kI...> all) {
+#pragma nounroll
+    for (int p = 0; p + 1 < 4 * kSlots; ++p) {
+        float rp[kSlots];
+        float vp[kSlots];
+        float app = 0.0F;
+        (quad_load_row<kSlots, kI>(a, v, p, rp, vp, app), ...);
+        (quad_rotate<kSlots, kI>(a, v, l, p, active, threshold, rp, vp, app, all), ...);
+        (quad_store_row<kSlots, kI>(a, v, l, p, rp, vp, app, all), ...);
+    }
+}
+
+// Eigenpairs in the stable descending order of the diagonal.  Every lane
+// walks a column of V in row order (the lane exchanges bring the other
+// lanes' rows), then writes its own rows of the canonical vector: a few
+// percent of the solver's instructions, and no LDS, whose staging of 16
+// problems would halve the wavefronts per compute unit.
+template <int kSlots, int kC, int... kI>
+__device__ __forceinline__ void quad_output_column(const float (&v)[kSlots][4 * kSlots],
+                                                   const float (&diag)[4 * kSlots], int l,
+                                                   bool valid, int n, int rank_limit, int stride,
+                                                   float* __restrict__ vectors, float* __restrict__ values,
+                                                   std::integer_sequence<int, kI...>) {
+    const float dr = diag[kC];
+    int rank = 0;
+    ((rank += kI < n && (diag[kI] > dr || (kI < kC && !(dr > diag[kI]))) ? 1 : 0), ...);
+    float norm_squared = 0.0F;
+    float max_abs = 0.0F;
+    float pivot = quad_lane<0>(v[0][kC]);
+    const auto add = [&](float value, bool held) {
+        if (held) {
+            norm_squared = norm_squared + value * value;
+            const float value_abs = fabsf(value);
+            if (value_abs > max_abs) {
+                max_abs = value_abs;
+                pivot = value;
+            }
+        }
+    };
+    (add(quad_lane<kI % 4>(v[kI / 4][kC]), kI < n), ...);
+    float scale = 1.0F;
+    const bool rescale = norm_squared > FLT_MIN;
+    if (rescale) {
+        scale = 1.0F / sqrtf(norm_squared);
+        if (pivot < 0.0F) {
+            scale = -scale;
+        }
+    }
+    if (valid && kC < n && rank < rank_limit) {
+#pragma unroll
+        for (int k = 0; k < kSlots; ++k) {
+            const int r = 4 * k + l;
+            if (r < n) {
+                vectors[static_cast<size_t>(rank) * stride + r] = rescale ? v[k][kC] * scale : v[k][kC];
+            }
+        }
+        if (l == 0) {
+            values[rank] = dr;
+        }
+    }
+}
+
+template <int kSlots, int... kI>
+__device__ __forceinline__ void quad_output(const float (&a)[kSlots][4 * kSlots],
+                                            const float (&v)[kSlots][4 * kSlots], int l, bool valid, int n,
+                                            int rank_limit, int stride, float* __restrict__ vectors,
+                                            float* __restrict__ values, std::integer_sequence<int, kI...> all) {
+    const float diag[] = {quad_lane<kI % 4>(a[kI / 4][kI])...};
+    (quad_output_column<kSlots, kI>(v, diag, l, valid, n, rank_limit, stride, vectors, values, all), ...);
+}
+
+template <int kSlots>
+__global__ __launch_bounds__(64) void jacobi_quad_kernel(
     StageDesc d, const int* __restrict__ group_count_dev, int problem_stride,
     const int* __restrict__ group_flags, const int* __restrict__ problem_dims,
     const float* __restrict__ problems, float* __restrict__ eigenvalues,
     float* __restrict__ vectors, int* __restrict__ status) {
+    constexpr int kN = 4 * kSlots;
+    constexpr int kPerWave = 16;
     const int problem_count = *group_count_dev * d.models;
-    constexpr int kPerWave = kLP >= 64 ? 1 : 64 / kLP;
-    constexpr int kStride = kLP + 1;
-    extern __shared__ float s_jacobi[];
-    __shared__ int s_order[kPerWave][kLP];
-    __shared__ float s_reduce[2];
-
-    const int sub = threadIdx.x / kLP;
-    const int r = threadIdx.x % kLP;
+    if (static_cast<int>(blockIdx.x) * kPerWave >= problem_count) {
+        return;
+    }
+    const int sub = threadIdx.x / 4;
+    const int l = threadIdx.x % 4;
     const int problem = blockIdx.x * kPerWave + sub;
     const int group = problem / d.models;
     bool valid = problem < problem_count;
@@ -53,53 +295,47 @@ __global__ __launch_bounds__(128) void jacobi_kernel(
         valid = (group_flags[group] & kFlagModelled) != 0;
         n = problem_dims[group];
     }
-    float* m = s_jacobi + static_cast<size_t>(sub) * 2 * kLP * kStride;
-    float* v = m + kLP * kStride;
     const float* in = problems + static_cast<size_t>(problem) * problem_stride * problem_stride;
-    // Maximum over the problem's lanes (all threads of the block call it).
-    const auto problem_max = [&](float value) {
-        for (int offset = (kLP < 64 ? kLP : 64) / 2; offset >= 1; offset >>= 1) {
-            value = fmaxf(value, __shfl_xor(value, offset, kLP < 64 ? kLP : 64));
-        }
-        if constexpr (kLP > 64) {
-            __syncthreads();
-            if ((threadIdx.x & 63) == 0) {
-                s_reduce[threadIdx.x >> 6] = value;
+    float a[kSlots][kN];
+    float v[kSlots][kN];
+    float scale = 0.0F;
+#pragma unroll
+    for (int k = 0; k < kSlots; ++k) {
+        const int r = 4 * k + l;
+#pragma unroll
+        for (int c = 0; c < kN; ++c) {
+            float value = 0.0F;
+            if (valid && r < n && c < n) {
+                value = in[r * problem_stride + c];
+                scale = fmaxf(scale, fabsf(value));
             }
-            __syncthreads();
-            value = fmaxf(s_reduce[0], s_reduce[1]);
+            a[k][c] = value;
+            v[k][c] = r == c ? 1.0F : 0.0F;
         }
-        return value;
-    };
-
-    float row_max = 0.0F;
-    for (int c = 0; c < kLP; ++c) {
-        float value = 0.0F;
-        if (valid && r < n && c < n) {
-            value = in[r * problem_stride + c];
-            row_max = fmaxf(row_max, fabsf(value));
-        }
-        m[r * kStride + c] = value;
-        v[r * kStride + c] = (r == c) ? 1.0F : 0.0F;
     }
-    row_max = problem_max(row_max);
-    const float matrix_scale = row_max > 1.0F ? row_max : 1.0F;
-    const float threshold = (64.0F * FLT_EPSILON) * matrix_scale;
-    __syncthreads();
-
+    scale = fmaxf(scale, xor16<1>(scale));
+    scale = fmaxf(scale, xor16<2>(scale));
+    const float threshold = (64.0F * FLT_EPSILON) * (scale > 1.0F ? scale : 1.0F);
     const auto offdiag_max = [&]() {
         float value = 0.0F;
-        if (r < n) {
-            for (int c = r + 1; c < n; ++c) {
-                value = fmaxf(value, fabsf(m[r * kStride + c]));
+#pragma unroll
+        for (int k = 0; k < kSlots; ++k) {
+#pragma unroll
+            for (int c = 0; c < kN; ++c) {
+                if (c / 4 == k) {
+                    value = fmaxf(value, l == c % 4 ? 0.0F : fabsf(a[k][c]));
+                } else {
+                    value = fmaxf(value, fabsf(a[k][c]));
+                }
             }
         }
-        return problem_max(value);
+        value = fmaxf(value, xor16<1>(value));
+        return fmaxf(value, xor16<2>(value));
     };
-
     bool done = !valid || n <= 1;
     bool converged = true;
     int sweeps = 0;
+#pragma nounroll
     for (int sweep = 0; sweep < d.max_sweeps; ++sweep) {
         if (!done) {
             sweeps = sweep + 1;
@@ -111,75 +347,266 @@ __global__ __launch_bounds__(128) void jacobi_kernel(
         if (__all(done)) {
             break;
         }
-        // With one problem per block its n bounds the pairs; with several
-        // per wavefront every lane walks all kLP (the barriers are shared).
-        const int pairs_n = kPerWave == 1 ? n : kLP;
-        for (int p = 0; p + 1 < pairs_n; ++p) {
-            for (int q = p + 1; q < pairs_n; ++q) {
-                bool rotate = !done && q < n;
-                float apq = 0.0F;
-                if (rotate) {
-                    apq = m[p * kStride + q];
-                    rotate = fabsf(apq) > threshold;
-                }
-                float c = 1.0F;
-                float s = 0.0F;
-                float new_pp = 0.0F;
-                float new_qq = 0.0F;
-                float new_rp = 0.0F;
-                float new_rq = 0.0F;
-                float new_vp = 0.0F;
-                float new_vq = 0.0F;
-                if (rotate) {
-                    // jacobi_rotate (linalg.cpp:153-202).
-                    const float app = m[p * kStride + p];
-                    const float aqq = m[q * kStride + q];
-                    const float tau = (aqq - app) / (2.0F * apq);
-                    const float tau_abs = fabsf(tau);
-                    const float t_abs = 1.0F / (tau_abs + sqrtf(1.0F + (tau * tau)));
-                    const float t = tau < 0.0F ? -t_abs : t_abs;
-                    c = 1.0F / sqrtf(1.0F + (t * t));
-                    s = t * c;
-                    const float cc = c * c;
-                    const float ss = s * s;
-                    const float cs = c * s;
-                    const float two_cs = 2.0F * cs;
-                    new_pp = ((cc * app) - (two_cs * apq)) + (ss * aqq);
-                    new_qq = ((ss * app) + (two_cs * apq)) + (cc * aqq);
-                    if (r < n && r != p && r != q) {
-                        const float arp = m[r * kStride + p];
-                        const float arq = m[r * kStride + q];
-                        new_rp = (c * arp) - (s * arq);
-                        new_rq = (s * arp) + (c * arq);
-                    }
-                    if (r < n) {
-                        const float vrp = v[r * kStride + p];
-                        const float vrq = v[r * kStride + q];
-                        new_vp = (c * vrp) - (s * vrq);
-                        new_vq = (s * vrp) + (c * vrq);
-                    }
-                }
-                __syncthreads();
-                if (rotate) {
-                    if (r < n && r != p && r != q) {
-                        m[r * kStride + p] = new_rp;
-                        m[p * kStride + r] = new_rp;
-                        m[r * kStride + q] = new_rq;
-                        m[q * kStride + r] = new_rq;
-                    }
-                    if (r == 0) {
-                        m[p * kStride + p] = new_pp;
-                        m[q * kStride + q] = new_qq;
-                        m[p * kStride + q] = 0.0F;
-                        m[q * kStride + p] = 0.0F;
-                    }
-                    if (r < n) {
-                        v[r * kStride + p] = new_vp;
-                        v[r * kStride + q] = new_vq;
-                    }
-                }
-                __syncthreads();
+        quad_sweep<kSlots>(a, v, l, !done, threshold, std::make_integer_sequence<int, kN>{});
+    }
+    const float final_off = offdiag_max();
+    if (!done) {
+        sweeps = d.max_sweeps;
+        converged = final_off <= 8.0F * threshold;
+    }
+    quad_output<kSlots>(a, v, l, valid, n, d.rank, problem_stride,
+                        vectors + static_cast<size_t>(problem) * d.rank * problem_stride,
+                        eigenvalues + static_cast<size_t>(problem) * d.rank,
+                        std::make_integer_sequence<int, kN>{});
+    if (valid && l == 0) {
+        status[problem] = sweeps | (converged ? 0 : (1 << 16));
+    }
+}
+
+// Larger problems, 64 / kLP per wavefront: lane x holds rows x (and x + 64,
+// kRows = 2).  A lives in LDS, both symmetric copies of an entry kept equal;
+// the running entries A[r][p], the diagonal and V stay in registers.  The
+// next column's entries are read one rotation ahead (only the row of the
+// current q changes in between, and its entry comes from the lane of row
+// q + 1), so a rotation waits for its pivot and its arithmetic only: no
+// barriers, no LDS round trip.  V takes a row's rotations after the row is
+// finished, from a log (lane q holds rotation (p, q)), so that every register
+// index is a constant.  Entries of row p are junk while it runs (see above);
+// rows and columns past n are zero and never rotate.  LDS holds A alone: a
+// 100-row problem takes 40400 bytes, four per compute unit.  Bound by the
+// chain of a rotation (pivot, divide, roots, pivot).  Measured against one
+// workgroup of a lane per row with A and V in LDS and two barriers a
+// rotation: 983 problems of 100 rows 57.5 -> 16.5 ms, 1.4 k of 60 rows 8.95
+// -> 4.50 ms.
+constexpr float kNoRotation = 2.0F;  // log entry: a rotation's c is at most 1
+
+__host__ __device__ inline int jacobi_row_stride(int problem_stride) { return problem_stride | 1; }
+__host__ __device__ inline size_t jacobi_problem_floats(int problem_stride) {
+    return static_cast<size_t>(problem_stride) * jacobi_row_stride(problem_stride);
+}
+
+// LDS accesses of one wavefront stay in program order; the compiler has to
+// keep them there.
+__device__ inline void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Value of row q (uniform) of the problem, one register per row.
+template <int kLP, int kRows> __device__ inline float row_value(const float (&v)[kRows], int q, bool upper) {
+    if constexpr (kLP == 32) {
+        const int lo = __builtin_amdgcn_readlane(__builtin_bit_cast(int, v[0]), q);
+        const int hi = __builtin_amdgcn_readlane(__builtin_bit_cast(int, v[0]), 32 + q);
+        return __builtin_bit_cast(float, upper ? hi : lo);
+    } else if constexpr (kRows == 2) {
+        const int lo = __builtin_amdgcn_readlane(__builtin_bit_cast(int, v[0]), q & 63);
+        const int hi = __builtin_amdgcn_readlane(__builtin_bit_cast(int, v[1]), q & 63);
+        return __builtin_bit_cast(float, q < 64 ? lo : hi);
+    } else {
+        return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v[0]), q));
+    }
+}
+
+template <int kLP, int kRows>
+__global__ __launch_bounds__(64) void jacobi_wave_kernel(
+    StageDesc d, const int* __restrict__ group_count_dev, int problem_stride,
+    const int* __restrict__ group_flags, const int* __restrict__ problem_dims,
+    const float* __restrict__ problems, float* __restrict__ eigenvalues,
+    float* __restrict__ vectors, int* __restrict__ status) {
+    constexpr int kN = kLP * kRows;
+    constexpr int kPerWave = 64 / kLP;
+    extern __shared__ __attribute__((aligned(16))) float s_jacobi[];
+    const int problem_count = *group_count_dev * d.models;
+    if (static_cast<int>(blockIdx.x) * kPerWave >= problem_count) {
+        return;
+    }
+    const int sub = threadIdx.x / kLP;
+    const bool upper = sub != 0;
+    const int lane = threadIdx.x % kLP;
+    const int problem = blockIdx.x * kPerWave + sub;
+    const int group = problem / d.models;
+    bool valid = problem < problem_count;
+    int n = 0;
+    if (valid) {
+        valid = (group_flags[group] & kFlagModelled) != 0;
+        n = problem_dims[group];
+    }
+    const int stride = jacobi_row_stride(problem_stride);
+    float* m = s_jacobi + sub * jacobi_problem_floats(problem_stride);
+    const float* in = problems + static_cast<size_t>(problem) * problem_stride * problem_stride;
+    // Rows past the matrix (lanes x >= problem_stride) read row 0 and never
+    // write.
+    int row[kRows];
+    bool in_matrix[kRows];
+    float* mine[kRows];
+    float diag[kRows];
+    float v[kRows][kN];
+    float scale = 0.0F;
+#pragma unroll
+    for (int k = 0; k < kRows; ++k) {
+        row[k] = lane + k * 64;
+        in_matrix[k] = row[k] < problem_stride;
+        mine[k] = m + (in_matrix[k] ? row[k] : 0) * stride;
+        diag[k] = 0.0F;
+#pragma unroll
+        for (int c = 0; c < kN; ++c) {
+            v[k][c] = row[k] == c ? 1.0F : 0.0F;
+        }
+    }
+    // Rows of the input are read by the whole problem's lanes.
+    for (int r = 0; r < problem_stride; ++r) {
+        for (int c = lane; c < problem_stride; c += kLP) {
+            float value = 0.0F;
+            if (valid && r < n && c < n) {
+                value = in[r * problem_stride + c];
+                scale = fmaxf(scale, fabsf(value));
             }
+            m[r * stride + c] = value;
+        }
+    }
+    for (int offset = kLP / 2; offset >= 1; offset >>= 1) {
+        scale = fmaxf(scale, __shfl_xor(scale, offset, kLP));
+    }
+    const float threshold = (64.0F * FLT_EPSILON) * (scale > 1.0F ? scale : 1.0F);
+    wave_lds_order();
+#pragma unroll
+    for (int k = 0; k < kRows; ++k) {
+        if (in_matrix[k]) {
+            diag[k] = mine[k][row[k]];
+        }
+    }
+    const int rows_max = __builtin_amdgcn_readfirstlane(wave_max_int(n));
+    const auto offdiag_max = [&]() {
+        float value = 0.0F;
+        wave_lds_order();
+#pragma unroll
+        for (int k = 0; k < kRows; ++k) {
+            if (row[k] < n) {
+                for (int c = 0; c < n; ++c) {
+                    value = fmaxf(value, c != row[k] ? fabsf(mine[k][c]) : 0.0F);
+                }
+            }
+        }
+        for (int offset = kLP / 2; offset >= 1; offset >>= 1) {
+            value = fmaxf(value, __shfl_xor(value, offset, kLP));
+        }
+        return value;
+    };
+    bool done = !valid || n <= 1;
+    bool converged = true;
+    int sweeps = 0;
+#pragma nounroll
+    for (int sweep = 0; sweep < d.max_sweeps; ++sweep) {
+        if (!done) {
+            sweeps = sweep + 1;
+        }
+        const float off = offdiag_max();
+        if (!done && off <= threshold) {
+            done = true;
+        }
+        if (__all(done)) {
+            break;
+        }
+#pragma nounroll
+        for (int p = 0; p + 1 < rows_max; ++p) {
+            float rp[kRows];
+            float column[kRows];
+            float log_c[kRows];
+            float log_s[kRows];
+#pragma unroll
+            for (int k = 0; k < kRows; ++k) {
+                rp[k] = mine[k][p];
+                column[k] = mine[k][p + 1];
+                log_c[k] = kNoRotation;
+                log_s[k] = 0.0F;
+            }
+            wave_lds_order();
+            float app = row_value<kLP, kRows>(diag, p, upper);
+            bool any = false;
+#pragma nounroll
+            for (int q = p + 1; q < rows_max; ++q) {
+                const int ahead = q + 1 < rows_max ? q + 1 : q;
+                float next[kRows];
+#pragma unroll
+                for (int k = 0; k < kRows; ++k) {
+                    next[k] = mine[k][ahead];
+                }
+                wave_lds_order();
+                const float apq = row_value<kLP, kRows>(rp, q, upper);
+                const float aqq = row_value<kLP, kRows>(diag, q, upper);
+                const bool rotate = !done && fabsf(apq) > threshold;
+                if (rotate) {
+                    any = true;
+                    const Rotation o = rotation_of(app, aqq, apq);
+                    app = o.new_pp;
+#pragma unroll
+                    for (int k = 0; k < kRows; ++k) {
+                        rotate_pair(o, rp[k], column[k]);
+                        if (in_matrix[k]) {
+                            mine[k][q] = column[k];
+                            m[q * stride + row[k]] = column[k];
+                        }
+                        const bool own = row[k] == q;
+                        rp[k] = own ? 0.0F : rp[k];
+                        diag[k] = own ? o.new_qq : diag[k];
+                        log_c[k] = own ? o.c : log_c[k];
+                        log_s[k] = own ? o.s : log_s[k];
+                    }
+                }
+                // Row q's entry of the next column is the one row q + 1 has
+                // just taken (the same value where nothing rotated).
+                const float fresh = row_value<kLP, kRows>(column, ahead, upper);
+#pragma unroll
+                for (int k = 0; k < kRows; ++k) {
+                    column[k] = row[k] == q && rotate ? fresh : next[k];
+                }
+                wave_lds_order();
+            }
+            // Row and column p.
+#pragma unroll
+            for (int k = 0; k < kRows; ++k) {
+                if (row[k] == p) {
+                    diag[k] = app;
+                } else if (in_matrix[k]) {
+                    mine[k][p] = rp[k];
+                    m[p * stride + row[k]] = rp[k];
+                }
+            }
+            wave_lds_order();
+            if (!__any(any)) {
+                continue;
+            }
+            float vp[kRows];
+#pragma unroll
+            for (int c = 0; c < kN; ++c) {
+                if (c == p) {
+#pragma unroll
+                    for (int k = 0; k < kRows; ++k) {
+                        vp[k] = pinned(v[k][c]);
+                    }
+                }
+            }
+#pragma unroll
+            for (int c = 1; c < kN; ++c) {
+                const Rotation o{row_value<kLP, kRows>(log_c, c, upper), row_value<kLP, kRows>(log_s, c, upper),
+                                 0.0F, 0.0F};
+                if (o.c != kNoRotation) {
+#pragma unroll
+                    for (int k = 0; k < kRows; ++k) {
+                        rotate_pair(o, vp[k], v[k][c]);
+                    }
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < kN; ++c) {
+                if (c == p) {
+#pragma unroll
+                    for (int k = 0; k < kRows; ++k) {
+                        v[k][c] = pinned(vp[k]);
+                    }
+                }
+            }
+            wave_lds_order();
         }
     }
     const float final_off = offdiag_max();
@@ -187,49 +614,50 @@ __global__ __launch_bounds__(128) void jacobi_kernel(
         sweeps = d.max_sweeps;
         converged = final_off <= 8.0F * threshold;
     }
-
-    // Stable descending order of the diagonal.
-    if (valid && r < n) {
-        const float dr = m[r * kStride + r];
-        int rank = 0;
-        for (int j = 0; j < n; ++j) {
-            const float dj = m[j * kStride + j];
-            rank += (dj > dr || (j < r && !(dr > dj))) ? 1 : 0;
+    // Stable descending order of the diagonal, then V, in A's place.  Lane x
+    // writes eigenpair x (the rank is at most 64, and at most n).
+    float* diagonal = m;
+    int* order = reinterpret_cast<int*>(m + problem_stride);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kRows; ++k) {
+        if (in_matrix[k]) {
+            diagonal[row[k]] = diag[k];
         }
-        s_order[sub][rank] = r;
     }
     __syncthreads();
-    if (valid && r < d.rank && r < n) {
-        const int col = s_order[sub][r];
-        float* vec_out = vectors + (static_cast<size_t>(problem) * d.rank + r) * problem_stride;
-        float norm_squared = 0.0F;
-        float max_abs = 0.0F;
-        int pivot = 0;
-        for (int i = 0; i < n; ++i) {
-            const float value = v[i * kStride + col];
-            const float square = value * value;
-            norm_squared = norm_squared + square;
-            const float value_abs = fabsf(value);
-            if (value_abs > max_abs) {
-                max_abs = value_abs;
-                pivot = i;
-            }
+    for (int r = lane; valid && r < n; r += kLP) {
+        const float dr = diagonal[r];
+        int rank = 0;
+        for (int j = 0; j < n; ++j) {
+            const float dj = diagonal[j];
+            rank += (dj > dr || (j < r && !(dr > dj))) ? 1 : 0;
         }
-        float scale = 1.0F;
-        const bool rescale = norm_squared > FLT_MIN;
-        if (rescale) {
-            scale = 1.0F / sqrtf(norm_squared);
-            if (v[pivot * kStride + col] < 0.0F) {
-                scale = -scale;
-            }
-        }
-        for (int i = 0; i < n; ++i) {
-            const float value = v[i * kStride + col];
-            vec_out[i] = rescale ? value * scale : value;
-        }
-        eigenvalues[static_cast<size_t>(problem) * d.rank + r] = m[col * kStride + col];
+        order[rank] = r;
     }
-    if (valid && r == 0) {
+    __syncthreads();
+    const bool writes = valid && lane < d.rank && lane < n;
+    const int col = writes ? order[lane] : 0;
+    const float value = writes ? diagonal[col] : 0.0F;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kRows; ++k) {
+        if (in_matrix[k]) {
+#pragma unroll
+            for (int c = 0; c < kN; ++c) {
+                if (c < problem_stride) {
+                    mine[k][c] = v[k][c];
+                }
+            }
+        }
+    }
+    __syncthreads();
+    if (writes) {
+        write_eigenvector(m, stride, n, col,
+                          vectors + (static_cast<size_t>(problem) * d.rank + lane) * problem_stride);
+        eigenvalues[static_cast<size_t>(problem) * d.rank + lane] = value;
+    }
+    if (valid && lane == 0) {
         status[problem] = sweeps | (converged ? 0 : (1 << 16));
     }
 }
@@ -644,31 +1072,31 @@ hipError_t launch_jacobi(const StageDesc& d, const int* group_count_dev, int pro
         return hipSuccess;
     }
     const int n = problem_stride;
-#define VNLBHIP_JACOBI(LP)                                                                      \
-    do {                                                                                        \
-        constexpr int kPer = LP >= 64 ? 1 : 64 / LP;                                            \
-        const size_t shared = static_cast<size_t>(kPer) * 2 * LP * (LP + 1) * sizeof(float);    \
-        hipLaunchKernelGGL(jacobi_kernel<LP>,                                                   \
-                           dim3(static_cast<unsigned>((problem_capacity + kPer - 1) / kPer)),   \
-                           dim3(LP > 64 ? LP : 64), shared, stream, d, group_count_dev,         \
-                           problem_stride, group_flags, problem_dims, problems, eigenvalues,    \
-                           vectors, status);                                                    \
-    } while (0)
+#define VNLBHIP_JACOBI(KERNEL, PER, SHARED)                                                     \
+    hipLaunchKernelGGL((KERNEL), dim3(static_cast<unsigned>((problem_capacity + PER - 1) / PER)), \
+                       dim3(64), SHARED, stream, d, group_count_dev, problem_stride,            \
+                       group_flags, problem_dims, problems, eigenvalues, vectors, status)
     if (n > 128) {
         return hipErrorInvalidValue;
     }
+    // Up to 16 rows a problem fits the registers of four lanes (512 of the
+    // lane's 512 registers would hold 20 rows); above, one or two problems per
+    // wavefront with A in LDS.
+    const size_t shared = jacobi_problem_floats(n) * sizeof(float);
     if (n <= 4) {
-        VNLBHIP_JACOBI(4);
+        VNLBHIP_JACOBI(jacobi_quad_kernel<1>, 16, 0);
     } else if (n <= 8) {
-        VNLBHIP_JACOBI(8);
+        VNLBHIP_JACOBI(jacobi_quad_kernel<2>, 16, 0);
+    } else if (n <= 12) {
+        VNLBHIP_JACOBI(jacobi_quad_kernel<3>, 16, 0);
     } else if (n <= 16) {
-        VNLBHIP_JACOBI(16);
+        VNLBHIP_JACOBI(jacobi_quad_kernel<4>, 16, 0);
     } else if (n <= 32) {
-        VNLBHIP_JACOBI(32);
+        VNLBHIP_JACOBI((jacobi_wave_kernel<32, 1>), 2, 2 * shared);
     } else if (n <= 64) {
-        VNLBHIP_JACOBI(64);
+        VNLBHIP_JACOBI((jacobi_wave_kernel<64, 1>), 1, shared);
     } else {
-        VNLBHIP_JACOBI(128);
+        VNLBHIP_JACOBI((jacobi_wave_kernel<64, 2>), 1, shared);
     }
 #undef VNLBHIP_JACOBI
     return hipGetLastError();
