@@ -531,6 +531,15 @@ struct DebugOutput {
 // at most kMaxParts, kDefaultParts unless the autotuner chose another count.
 constexpr int kMaxParts = 4;
 constexpr int kDefaultParts = 2;
+// Batches of at most this many anchors run the model (prepare, eigen solve,
+// filter) once over the groups of all their parts: the parts' group lists
+// are joined.  The model kernels of so few groups take the time of a group's
+// serial chain, not of their work, and a launch per part pays it again
+// (256x256x5 GrayS, 5.4 k anchors: 1134 us a pass with two model launches per
+// stage, 940 us with one; 717x403x7 uncoupled YUV, 57 k anchors: 9.79 ->
+// 9.56 ms).  Above, the first part's model covers the last part's paste scan
+// (150 k anchors: 16.1 ms against 16.2 without).
+constexpr int kJoinedAnchors = 1 << 16;
 
 struct vnlbhip_context {
     int device = 0;
@@ -1032,6 +1041,8 @@ void run_stage(vnlbhip_context& ctx, int stage, const vnlbhip_params& p, const f
         for (int h = 0; h <= parts; ++h) {
             part_frame[h] = frame_count * h / parts;
         }
+        // (A scratch call keeps the smaller buffers of separate lists.)
+        const bool joined = anchor_count <= kJoinedAnchors && !ctx.generation.arena.active;
         check(hipEventRecord(ctx.ready_event, stream), "hipEventRecord");
         check(hipStreamWaitEvent(ctx.side, ctx.ready_event, 0), "hipStreamWaitEvent");
 
@@ -1167,7 +1178,10 @@ void run_stage(vnlbhip_context& ctx, int stage, const vnlbhip_params& p, const f
                                              d_positions, d_active, max_anchors, ae - ab, d_dep, d_tcount,
                                              d_targets, anchor_count, ctx.side);
             });
-            untimed(ctx, "compact kernel", [&]() { return vnlbhip::launch_compact(d_active, ab, ae - ab, d_list + ab, d_group_count + h, ctx.side); });
+            untimed(ctx, "compact kernel", [&]() {
+                return vnlbhip::launch_compact(d_active, ab, ae - ab, joined ? d_list : d_list + ab,
+                                               joined ? d_group_count : d_group_count + h, ctx.side);
+            });
             check(hipEventRecord(ctx.paste_event[h], ctx.side), "hipEventRecord");
         }
 
@@ -1188,7 +1202,7 @@ void run_stage(vnlbhip_context& ctx, int stage, const vnlbhip_params& p, const f
         // The group count of a part is read on the device (the compaction
         // wrote it); grids and buffers are sized by the largest part's anchor
         // count, so the host never waits for the paste scans.
-        int part_capacity = 0;
+        int part_capacity = joined ? anchor_count : 0;
         for (int h = 0; h < parts; ++h) {
             part_capacity = std::max(part_capacity, grid.offsets[static_cast<size_t>(part_frame[h + 1])] -
                                                         grid.offsets[static_cast<size_t>(part_frame[h])]);
@@ -1259,7 +1273,11 @@ void run_stage(vnlbhip_context& ctx, int stage, const vnlbhip_params& p, const f
             check(hipStreamWaitEvent(stream, ctx.paste_event[h], 0), "hipStreamWaitEvent");
             const int ab = grid.offsets[static_cast<size_t>(part_frame[h])];
             const int ae = grid.offsets[static_cast<size_t>(part_frame[h + 1])];
-            run_model(d_list + ab, d_group_count + h, ae - ab);
+            if (!joined) {
+                run_model(d_list + ab, d_group_count + h, ae - ab);
+            } else if (h + 1 == parts) {
+                run_model(d_list, d_group_count, anchor_count);
+            }
         }
         if (lists != nullptr && !ctx.sizing) {
             *lists->anchor_count = anchor_count;
