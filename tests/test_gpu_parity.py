@@ -194,3 +194,42 @@ def test_invalid_parameters_raise(gpu):
     p = StageParameters(sigma=0.1, rank=32, similar=16, patch_time=1)
     with pytest.raises(vnlbhip.VNLBError, match="group_size must cover the effective VNLB rank"):
         gpu.stage(BASIC, p, noisy)
+
+
+@pytest.mark.parametrize("channels,extra", [
+    # Groups of one round of samples, the tile over the basis (YUV rank 16).
+    (3, dict(group_size=16, rank=16)),
+    # Groups that widen past one round there (no tile), and past one round of a tile of its own.
+    (3, dict(group_size=16, rank=16, tau=200000)),
+    (3, dict(group_size=10, rank=2, tau=200000)),
+    (1, dict(group_size=8, rank=8, tau=200000)),
+    (3, dict(group_size=9, rank=4, tau=200000, chroma=0)),
+    # More samples than a round by the group size itself.
+    (1, dict(group_size=40, rank=12)),
+    # Windows too wide for a tile, single-sample groups, one to four patch frames.
+    (3, dict(group_size=16, rank=4, bm_range=18)),
+    (1, dict(group_size=1, rank=1)),
+    (1, dict(group_size=16, rank=6, patch_time=1)),
+    (1, dict(group_size=16, rank=6, patch_time=3)),
+    (1, dict(group_size=16, rank=6, patch_time=4)),
+    # Unit aggregation window, rank 0.
+    (3, dict(group_size=16, rank=0, weight_gamma=0.0))])
+def test_aggregation_paths(gpu, oracle_lib, channels, extra):
+    """Every way a group's samples reach the accumulators, on a width that is
+    no multiple of a memory line.  Both sides add the same float products in
+    double; the weights agree to 1e-6 relative (see above) and samples stay
+    below 2 in magnitude, so the weighted means differ by at most 2 * 2e-6 and
+    a float rounding: 5e-6."""
+    noisy, _ = synth.make_clip(61, 45, 5, channels, sigma8=5, seed=123, motion="subpixel")
+    args = dict(dict(sigma=15, block_size=8, block_step=5, bm_range=7, patch_time=2, radius=1, tau=0), **extra)
+    bp, fp = parse_stage_parameters(BASIC, args), parse_stage_parameters(FINAL, args)
+    print(f"[parity] aggregation {channels} {extra}", flush=True)
+    want_basic, _ = oracle_lib.stage(BASIC, bp, noisy, flags=oracle_lib.ACCUM_DOUBLE, threads=4)
+    want_final, _ = oracle_lib.stage(FINAL, fp, noisy, want_basic, flags=oracle_lib.ACCUM_DOUBLE, threads=4)
+    basic = gpu.stage(BASIC, bp, _dev(noisy))
+    if args["tau"] > 0:
+        stats = gpu.stats()
+        assert stats["retained"] > 1.5 * args["group_size"] * stats["groups"]
+    final = gpu.stage(FINAL, fp, _dev(noisy), _dev(want_basic))
+    for got, want in ((basic, want_basic), (final, want_final)):
+        assert np.abs(got.cpu().numpy().reshape(want.shape) - want).max() <= 5e-6

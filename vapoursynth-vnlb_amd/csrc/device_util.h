@@ -7,6 +7,13 @@
 
 namespace vnlbhip {
 
+// A value the compiler has to have in a register here: keeps it from turning
+// a chain of cases over one register array into an indexed array in memory.
+__device__ __forceinline__ float pinned(float v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
 // XCD-aware work distribution (kXcds, counters: common.h).  The GPU
 // dispatches the workgroups of a launch round-robin over its 8 XCDs (block b
 // on XCD b % 8), and each XCD has its own L2: work that shares data

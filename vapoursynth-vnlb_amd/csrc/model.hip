@@ -122,13 +122,6 @@ template <int kLane> __device__ inline float quad_lane(float v) {
         float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), kLane * 0x55, 0xF, 0xF, true));
 }
 
-// A value the compiler has to have in a register here: keeps it from turning
-// a chain of cases over one register array into an indexed array in memory.
-__device__ __forceinline__ float pinned(float v) {
-    asm volatile("" : "+v"(v));
-    return v;
-}
-
 // Problems of at most 4 kSlots (<= 16) rows: four lanes per problem, sixteen
 // problems per wavefront, A and V in registers; lane l holds the rows
 // l, l + 4, ... (slot k is row 4 k + l).  Bound by instruction issue: a
