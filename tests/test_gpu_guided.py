@@ -15,7 +15,7 @@ import torch
 import vnlbhip
 import workloads
 from vnlbhip import synth
-from vnlbhip.params import BASIC, FINAL
+from vnlbhip.params import BASIC, FINAL, parse_stage_parameters
 
 from test_gpu_parity import _check_output, _compare_frame, _dev
 
@@ -142,3 +142,24 @@ def test_guided_rejects_a_mismatched_field(gpu):
         gpu.set_search_offsets(None)
     with pytest.raises(vnlbhip.VNLBError):
         gpu.set_search_offsets(torch.zeros((2, 2), dtype=torch.int16, device="cuda:0"))
+
+
+@pytest.mark.parametrize("bm_range,radius,patch_size", [(3, 1, 8), (6, 2, 5), (10, 1, 16), (18, 3, 8)])
+def test_guided_window_sizes(gpu, oracle_lib, bm_range, radius, patch_size):
+    """Guided match lists bit for bit at the edges of the matcher's staging: a
+    row of candidates per thread and two of them, windows no multiple of four
+    wide, and (37x37x7) planes that leave no room for 16-byte rows in LDS."""
+    noisy, _ = synth.make_clip(70, 62, 2 * radius + 3, 1, sigma8=15, seed=40 + bm_range, motion="subpixel")
+    bp = parse_stage_parameters(BASIC, dict(sigma=15, block_size=patch_size, block_step=14, group_size=12,
+                                            bm_range=bm_range, patch_time=2, radius=radius, rank=4, tau=0))
+    field, temporal = _field(noisy, bp, seed=bm_range)
+    print(f"[guided] window {2 * bm_range + 1}, radius {radius}", flush=True)
+    dev_field = torch.from_numpy(field).to("cuda:0")
+    try:
+        oracle_lib.set_search_offsets(field, temporal)
+        gpu.set_search_offsets(dev_field)
+        _compare_frame(gpu, oracle_lib, BASIC, bp, noisy, None, radius)
+    finally:
+        gpu.set_search_offsets(None)
+        oracle_lib.set_search_offsets(None)
+    _compare_frame(gpu, oracle_lib, BASIC, bp, noisy, None, radius)

@@ -15,26 +15,20 @@
 #include "proposer.h"
 #include "select.h"
 
+#include <type_traits>
+
 namespace vnlbhip {
 namespace {
 
 constexpr int kMatchThreads = 256;
 
-// Row distance of 4 horizontally adjacent candidates against one reference
-// row, each added to its running distance in the reference's element order.
-template <int kP>
-__device__ inline void add_row_distance4(float (&distance)[4], const float* ref_row,
-                                         const float* cand_row) {
-    float values[kP + 3];
-#pragma unroll
-    for (int i = 0; i < kP + 3; ++i) {
-        values[i] = cand_row[i];
-    }
-    float ref[kP];
-#pragma unroll
-    for (int i = 0; i < kP; ++i) {
-        ref[i] = ref_row[i];
-    }
+// Row distance of 4 horizontally adjacent candidates (values[j ..]) against
+// one reference row, each added to its running distance in the reference's
+// element order.
+template <int kP, int kV>
+__device__ __forceinline__ void add_row_distance4(float (&distance)[4], const float* __restrict__ ref,
+                                                  const float (&values)[kV]) {
+    static_assert(kV >= kP + 3, "four candidates span P + 3 samples");
     if (kP == kLanes) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -55,12 +49,65 @@ __device__ inline void add_row_distance4(float (&distance)[4], const float* ref_
         }
     } else {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int i = 0; i < kP; ++i) {
 #pragma unroll
-            for (int i = 0; i < kP; ++i) {
+            for (int j = 0; j < 4; ++j) {
                 const float diff = ref[i] - values[j + i];
                 const float square = diff * diff;
                 distance[j] = distance[j] + square;
+            }
+        }
+    }
+}
+
+// The same with the samples in LDS (the proposing matcher's scans).
+template <int kP>
+__device__ inline void add_row_distance4(float (&distance)[4], const float* ref_row, const float* cand_row) {
+    float values[kP + 3];
+#pragma unroll
+    for (int i = 0; i < kP + 3; ++i) {
+        values[i] = cand_row[i];
+    }
+    float ref[kP];
+#pragma unroll
+    for (int i = 0; i < kP; ++i) {
+        ref[i] = ref_row[i];
+    }
+    add_row_distance4<kP, kP + 3>(distance, ref, values);
+}
+
+// One patch frame of kRows vertically times 4 horizontally adjacent
+// candidates: every region row is loaded once for the candidates of all
+// kRows rows.  region: the first candidate's patch row in LDS (kWide: 16-byte
+// aligned rows); ref: the reference patch's first row, in the clip (uniform
+// rows: scalar loads) or in LDS.
+template <int kP, int kRows, bool kWide>
+__device__ __forceinline__ void add_patch_distances(float (&distance)[kRows][4], const float* __restrict__ ref,
+                                                    int ref_pitch, const float* region, int pitch) {
+    constexpr int kV = (kP + 3 + 3) / 4 * 4;
+#pragma unroll
+    for (int y = 0; y < kP + kRows - 1; ++y) {
+        float values[kV];
+        if constexpr (kWide) {
+            const float4* v4 = reinterpret_cast<const float4*>(region + y * pitch);
+#pragma unroll
+            for (int q = 0; q < kV / 4; ++q) {
+                const float4 v = v4[q];
+                values[4 * q + 0] = v.x;
+                values[4 * q + 1] = v.y;
+                values[4 * q + 2] = v.z;
+                values[4 * q + 3] = v.w;
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < kV; ++i) {
+                values[i] = i < kP + 3 ? region[y * pitch + i] : 0.0F;
+            }
+        }
+#pragma unroll
+        for (int rr = 0; rr < kRows; ++rr) {
+            if (y - rr >= 0 && y - rr < kP) {
+                add_row_distance4<kP, kV>(distance[rr], ref + (y - rr) * ref_pitch, values);
             }
         }
     }
@@ -83,6 +130,20 @@ __host__ __device__ inline int region_floats(int window, int patch, int temporal
     return (guided ? temporal * patch_time : temporal + patch_time - 1) * side * side + 8;
 }
 
+// The exhaustive matcher's region: rows of a 16-byte multiple that hold the
+// four samples past the last group of four candidates, and one row more (the
+// second of a pair of candidate rows may lie past the window).  Where that
+// exceeds the LDS of a workgroup, rows as narrow as region_floats has them.
+__host__ __device__ inline int region_pitch(int window, int patch, bool wide) {
+    return wide ? (window + 3) / 4 * 4 + (patch + 3 + 3) / 4 * 4 - 4 : window + patch - 1;
+}
+__host__ __device__ inline int match_region_floats(int window, int patch, int temporal, int patch_time, bool guided,
+                                                   bool wide) {
+    const int rows = (guided ? temporal * patch_time : temporal + patch_time - 1) * (window + patch - 1);
+    return wide ? ((rows + 1) * region_pitch(window, patch, true) + 3) / 4 * 4
+                : region_floats(window, patch, temporal, patch_time, guided) + window + patch - 1;
+}
+
 // Candidate distances of a full window: window^2 per scheduled frame.
 __host__ __device__ inline int window_candidates(const StageDesc& d) {
     return d.search_window * d.search_window * (d.search_bwd + d.search_fwd + 1);
@@ -96,11 +157,17 @@ __host__ __device__ inline int selection_entries(const StageDesc& d) {
 }
 
 // Distances (scan order) with the search region staged in LDS one channel
-// at a time; each thread owns 4 horizontally adjacent candidates of one
-// row so every loaded sample feeds 4 distances.  The per-candidate order of
+// at a time; each thread owns 4 horizontally adjacent candidates of one row,
+// or of two where one row each would fill the workgroup more than once, so
+// every loaded sample feeds 4 or 8 distances.  The per-candidate order of
 // additions is exactly that of the CPU scan: channel, frame offset, row,
-// column.
-template <int kP, bool kGuided>
+// column (three roundings per element, no fused form).  Bound by those
+// instructions (a 19x19x5 window of 384-sample patches takes 32.5 k vector
+// instructions of a wavefront) with the LDS reads beside them: sharing a row
+// between two candidate rows, 16-byte reads, the reference patch from scalar
+// loads and the staging by rows took 201 k anchors of a 1280x720 YUV clip
+// (mean of both stages) from 8.6 to 7.3 ms.
+template <int kP, bool kGuided, bool kWide>
 __global__ __launch_bounds__(kMatchThreads) void match_kernel(
     StageDesc d, const float* __restrict__ source, const uint32_t* __restrict__ anchors,
     int anchor_count, int* __restrict__ counts, uint32_t* __restrict__ positions,
@@ -109,7 +176,6 @@ __global__ __launch_bounds__(kMatchThreads) void match_kernel(
     // Guided search: the window origin of each scheduled frame.
     __shared__ int s_frame_x_low[kMaxTemporal];
     __shared__ int s_frame_y_low[kMaxTemporal];
-    __shared__ float s_ref[kMaxDim];
     __shared__ unsigned s_hist[256];
     __shared__ int s_int[16];
     __shared__ int s_scan[8];
@@ -136,7 +202,6 @@ __global__ __launch_bounds__(kMatchThreads) void match_kernel(
     const bool final_stage = d.stage == kFinal;
     const int match_channels = final_stage ? d.channels : 1;
     constexpr int P = kP;
-    constexpr int area = kP * kP;
 
     int t_low = 0;
     int t_high = 0;
@@ -179,81 +244,126 @@ __global__ __launch_bounds__(kMatchThreads) void match_kernel(
         }
     }
     const int rframes = guided ? nt * d.patch_time : nt + d.patch_time - 1;
-    const int plane = rrows * rcols;
-    const int region_size = rframes * plane;
+    const int pitch = region_pitch(d.search_window, P, kWide);
+    const int plane = rrows * pitch;
 
     float* s_region = s_dyn;
-    float* s_dist = s_dyn + region_floats(d.search_window, P, d.search_bwd + d.search_fwd + 1,
-                                          d.patch_time, guided);
+    float* s_dist = s_dyn + match_region_floats(d.search_window, P, d.search_bwd + d.search_fwd + 1,
+                                                d.patch_time, guided, kWide);
     // Selection scratch after the candidate distances.
     float* s_sel_dist = s_dist + window_candidates(d);
     int* s_sel_index = reinterpret_cast<int*>(s_sel_dist + selection_entries(d));
     int* s_sel_rank = s_sel_index + selection_entries(d);
-
-    // Reference patch [c][t][y][x] (load_reference_patch_* core.cpp:1152-1198).
-    const int ref_len = match_channels * d.patch_time * area;
-    for (int i = threadIdx.x; i < ref_len; i += blockDim.x) {
-        const int c = i / (d.patch_time * area);
-        const int rem = i - c * d.patch_time * area;
-        const int t = rem / area;
-        const int yx = rem - t * area;
-        const int y = yx / P;
-        const int x = yx - y * P;
-        s_ref[i] = video_at(source, d, ax + x, ay + y, af + t, c);
-    }
-    for (int i = region_size + threadIdx.x; i < region_size + 8; i += blockDim.x) {
-        s_region[i] = 0.0F;
-    }
+    float* s_ref = reinterpret_cast<float*>(s_sel_rank + selection_entries(d));
 
     const int groups_x = (nx + 3) >> 2;
-    const int items = nt * ny * groups_x;
-    for (int ch = 0; ch < match_channels; ++ch) {
-        __syncthreads();
-        for (int i = threadIdx.x; i < region_size; i += blockDim.x) {
-            const int fr = i / plane;
-            const int rem = i - fr * plane;
-            const int ry = rem / rcols;
-            const int rx = rem - ry * rcols;
-            if (guided) {
-                const int ti = fr / d.patch_time;
-                const int t = fr - ti * d.patch_time;
-                s_region[i] = video_at(source, d, s_frame_x_low[ti] + rx, s_frame_y_low[ti] + ry,
-                                       scheduled_frame(af, t_low, t_high, ti) + t, ch);
-            } else {
-                s_region[i] = video_at(source, d, x_low + rx, y_low + ry, t_low + fr, ch);
-            }
+    const bool paired = nt * ny * groups_x > kMatchThreads;
+    if (!paired) {
+        // Few candidates per thread and few wavefronts to cover a scalar
+        // load's latency: the reference patch [c][t][y][x] in LDS.
+        for (int i = threadIdx.x; i < match_channels * d.patch_dim; i += blockDim.x) {
+            const int ct = i / (P * P);
+            const int yx = i - ct * P * P;
+            const int c = ct / d.patch_time;
+            s_ref[i] = video_at(source, d, ax + yx % P, ay + yx / P, af + ct - c * d.patch_time, c);
         }
-        __syncthreads();
+    }
+    const size_t frame_stride = static_cast<size_t>(d.channels) * d.height * d.width;
+    // Half a wavefront stages a row of the region.
+    constexpr int kRowLanes = 32;
+    constexpr int kRowBatch = 8;
+    const int row_lane = threadIdx.x % kRowLanes;
+    const auto scan = [&](auto rows_per, int ch) {
+        constexpr int kRows = decltype(rows_per)::value;
+        const int ny_items = (ny + kRows - 1) / kRows;
+        const int items = nt * ny_items * groups_x;
+        // The reference patch of this channel: uniform rows of the clip
+        // (load_reference_patch_* core.cpp:1152-1198).
+        const float* __restrict__ ref =
+            source + ((static_cast<size_t>(af) * d.channels + ch) * d.height + ay) * d.width + ax;
         for (int item = threadIdx.x; item < items; item += blockDim.x) {
-            const int gx = item % groups_x;
-            const int rest = item / groups_x;
-            const int yy = rest % ny;
-            const int ti = rest / ny;
-            const int xx0 = gx * 4;
+            const int rest = item / ny_items;
+            const int yy = (item - rest * ny_items) * kRows;
+            const int ti = rest / groups_x;
+            const int xx0 = (rest - ti * groups_x) * 4;
             const int frame = scheduled_frame(af, t_low, t_high, ti);
             const int base_c = ti * per_frame + yy * nx + xx0;
             const int valid = nx - xx0 < 4 ? nx - xx0 : 4;
-            float dist[4];
+            float dist[kRows][4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                dist[j] = (ch == 0 || j >= valid) ? 0.0F : s_dist[base_c + j];
+            for (int rr = 0; rr < kRows; ++rr) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    dist[rr][j] =
+                        (ch == 0 || j >= valid || yy + rr >= ny) ? 0.0F : s_dist[base_c + rr * nx + j];
+                }
             }
             for (int t = 0; t < d.patch_time; ++t) {
-                const float* region_plane =
-                    s_region + (guided ? ti * d.patch_time + t : frame - t_low + t) * plane;
-                const float* ref_plane = s_ref + (ch * d.patch_time + t) * area;
-#pragma unroll
-                for (int y = 0; y < P; ++y) {
-                    add_row_distance4<kP>(dist, ref_plane + y * P,
-                                          region_plane + (yy + y) * rcols + xx0);
+                const int fr = guided ? ti * d.patch_time + t : frame - t_low + t;
+                const float* region = s_region + fr * plane + yy * pitch + xx0;
+                if constexpr (kRows == 1) {
+                    add_patch_distances<kP, 1, kWide>(dist, s_ref + (ch * d.patch_time + t) * P * P, P, region,
+                                                      pitch);
+                } else {
+                    add_patch_distances<kP, kRows, kWide>(dist, ref + t * frame_stride, d.width, region, pitch);
                 }
             }
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                if (j < valid) {
-                    s_dist[base_c + j] = dist[j];
+            for (int rr = 0; rr < kRows; ++rr) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    if (j < valid && yy + rr < ny) {
+                        s_dist[base_c + rr * nx + j] = dist[rr][j];
+                    }
                 }
             }
+        }
+    };
+    for (int ch = 0; ch < match_channels; ++ch) {
+        __syncthreads();
+        for (int rx = row_lane; rx < rcols; rx += kRowLanes) {
+            int fr = 0;
+            int ry = threadIdx.x / kRowLanes;
+            // Batches of rows, their loads issued together.
+            while (fr < rframes) {
+                float value[kRowBatch];
+                int to[kRowBatch];
+#pragma unroll
+                for (int k = 0; k < kRowBatch; ++k) {
+                    while (ry >= rrows) {
+                        ry -= rrows;
+                        ++fr;
+                    }
+                    to[k] = -1;
+                    value[k] = 0.0F;
+                    if (fr < rframes) {
+                        int x0 = x_low;
+                        int y0 = y_low;
+                        int frame = t_low + fr;
+                        if (guided) {
+                            const int ti = fr / d.patch_time;
+                            x0 = s_frame_x_low[ti];
+                            y0 = s_frame_y_low[ti];
+                            frame = scheduled_frame(af, t_low, t_high, ti) + fr - ti * d.patch_time;
+                        }
+                        value[k] = video_at(source, d, x0 + rx, y0 + ry, frame, ch);
+                        to[k] = fr * plane + ry * pitch + rx;
+                    }
+                    ry += kMatchThreads / kRowLanes;
+                }
+#pragma unroll
+                for (int k = 0; k < kRowBatch; ++k) {
+                    if (to[k] >= 0) {
+                        s_region[to[k]] = value[k];
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        if (paired) {
+            scan(std::integral_constant<int, 2>{}, ch);
+        } else {
+            scan(std::integral_constant<int, 1>{}, ch);
         }
     }
     __syncthreads();
@@ -648,19 +758,34 @@ hipError_t launch_match(const StageDesc& d, const float* source,
     }
     const dim3 grid(static_cast<unsigned>(anchor_count));
     const dim3 block(kMatchThreads);
-    const size_t shared = match_shared_bytes(d, offsets != nullptr);
+    const bool guided = offsets != nullptr;
+    const int temporal = d.search_bwd + d.search_fwd + 1;
+    // Guided windows have a plane per scheduled and patch frame; wide rows may
+    // not fit beside them (unguided ones always do: at most 108 KB narrow).
+    const size_t others = match_shared_bytes(d, guided) -
+                          sizeof(float) * region_floats(d.search_window, d.patch, temporal, d.patch_time, guided);
+    const auto shared_bytes = [&](bool wide) {
+        return others + sizeof(float) * match_region_floats(d.search_window, d.patch, temporal, d.patch_time,
+                                                            guided, wide) +
+               sizeof(float) * d.dim;
+    };
+    constexpr size_t kMatchLds = 156 * 1024;  // 160 KB less the kernel's static arrays
+    const bool wide = shared_bytes(true) <= kMatchLds;
+    const size_t shared = shared_bytes(wide);
+#define VNLBHIP_MATCH(PV, GUIDED, WIDE)                                                          \
+    hipLaunchKernelGGL((match_kernel<PV, GUIDED, WIDE>), grid, block, shared, stream, d, source, \
+                       anchors, anchor_count, counts, positions, distances, offsets,             \
+                       offsets_temporal)
     switch (d.patch) {
-#define VNLBHIP_MATCH_CASE(PV)                                                                  \
-    case PV:                                                                                    \
-        if (offsets != nullptr) {                                                               \
-            hipLaunchKernelGGL((match_kernel<PV, true>), grid, block, shared, stream, d, source, \
-                               anchors, anchor_count, counts, positions, distances, offsets,   \
-                               offsets_temporal);                                               \
-        } else {                                                                                \
-            hipLaunchKernelGGL((match_kernel<PV, false>), grid, block, shared, stream, d, source,\
-                               anchors, anchor_count, counts, positions, distances, offsets,   \
-                               offsets_temporal);                                               \
-        }                                                                                       \
+#define VNLBHIP_MATCH_CASE(PV)                  \
+    case PV:                                    \
+        if (!guided) {                          \
+            VNLBHIP_MATCH(PV, false, true);     \
+        } else if (wide) {                      \
+            VNLBHIP_MATCH(PV, true, true);      \
+        } else {                                \
+            VNLBHIP_MATCH(PV, true, false);     \
+        }                                       \
         break;
         VNLBHIP_MATCH_CASE(1)
         VNLBHIP_MATCH_CASE(2)
@@ -679,6 +804,7 @@ hipError_t launch_match(const StageDesc& d, const float* source,
         VNLBHIP_MATCH_CASE(15)
         VNLBHIP_MATCH_CASE(16)
 #undef VNLBHIP_MATCH_CASE
+#undef VNLBHIP_MATCH
     default:
         return hipErrorInvalidValue;
     }
