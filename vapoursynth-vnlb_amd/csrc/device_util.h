@@ -195,6 +195,14 @@ __device__ inline float xor16(float value) {
     return __builtin_bit_cast(float, xor16_bits<kMask>(__builtin_bit_cast(int, value)));
 }
 
+template <int kMask>
+__device__ inline double xor16(double value) {
+    const uint64_t bits = __builtin_bit_cast(uint64_t, value);
+    const uint32_t lo = static_cast<uint32_t>(xor16_bits<kMask>(static_cast<int>(bits & 0xFFFFFFFFu)));
+    const uint32_t hi = static_cast<uint32_t>(xor16_bits<kMask>(static_cast<int>(bits >> 32)));
+    return __builtin_bit_cast(double, (static_cast<uint64_t>(hi) << 32) | lo);
+}
+
 // 64-bit value from lane (lane ^ kMask) of the wavefront: DPP within rows of
 // 16 lanes, ds_bpermute across rows.
 template <int kMask>

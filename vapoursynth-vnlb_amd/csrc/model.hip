@@ -900,157 +900,178 @@ __global__ __launch_bounds__(64) void jacobi_parallel_kernel(
     }
 }
 
-// fp64 re-solve of the flagged problems (cyclic Jacobi in double, the
-// reference's solver at its double instantiation, linalg.cpp:447-550: same
-// rotation, threshold 64 eps max(1, max|A|) with the double eps, stopping
-// rule, ordering and canonical vectors), results rounded to float.  One
-// problem per wavefront at a time, lane r owning row r; the list length is
-// read on the device, so no host round trip is needed.
+// The parallel ordering in double with the full-precision operations, for
+// the re-solve below (same layout and rounds as parallel_round).
+template <int kK, int kJ>
+__device__ __forceinline__ void rotate_columns_double(double (&a)[16], double (&v)[16], const double (&b)[16],
+                                                      double c, double sigma) {
+    constexpr int kHigh = kK >= 8 ? 8 : (kK >= 4 ? 4 : (kK >= 2 ? 2 : 1));
+    if constexpr ((kJ & kHigh) == 0) {
+        constexpr int kJJ = kJ ^ kK;
+        const double c0 = xor16<kJ>(c);
+        const double s0 = xor16<kJ>(sigma);
+        const double v0 = v[kJ];
+        const double v1 = v[kJJ];
+        a[kJ] = fma(s0, b[kJJ], c0 * b[kJ]);
+        a[kJJ] = fma(-s0, b[kJ], c0 * b[kJJ]);
+        v[kJ] = fma(s0, v1, c0 * v0);
+        v[kJJ] = fma(-s0, v0, c0 * v1);
+    }
+}
+
+template <int kK, int... kJ>
+__device__ __forceinline__ void parallel_round_double(double (&a)[16], double (&v)[16], int r, bool active,
+                                                      double threshold, std::integer_sequence<int, kJ...>) {
+    constexpr int kHigh = kK >= 8 ? 8 : (kK >= 4 ? 4 : (kK >= 2 ? 2 : 1));
+    const bool is_p = (r & kHigh) == 0;
+    const double partner_diag = xor16<kK>(a[0]);
+    const double partner_off = xor16<kK>(a[kK]);
+    const double app = is_p ? a[0] : partner_diag;
+    const double aqq = is_p ? partner_diag : a[0];
+    const double apq = is_p ? a[kK] : partner_off;
+    const bool rotate = active && fabs(apq) > threshold;
+    if (!__any(rotate)) {
+        return;
+    }
+    const double tau = (aqq - app) / (2.0 * (rotate ? apq : 1.0));
+    const double t_abs = 1.0 / (fabs(tau) + sqrt(1.0 + tau * tau));
+    const double t = tau < 0.0 ? -t_abs : t_abs;
+    const double c_rot = 1.0 / sqrt(1.0 + t * t);
+    const double s_rot = t * c_rot;
+    const double cc = c_rot * c_rot;
+    const double ss = s_rot * s_rot;
+    const double two_cs = 2.0 * (c_rot * s_rot);
+    const double new_pp = ((cc * app) - (two_cs * apq)) + (ss * aqq);
+    const double new_qq = ((ss * app) + (two_cs * apq)) + (cc * aqq);
+    const double c = rotate ? c_rot : 1.0;
+    const double sigma = rotate ? (is_p ? -s_rot : s_rot) : 0.0;
+    double b[16];
+    ((b[kJ] = fma(sigma, xor16<kK>(a[kJ ^ kK]), c * a[kJ])), ...);
+    (rotate_columns_double<kK, kJ>(a, v, b, c, sigma), ...);
+    a[0] = rotate ? (is_p ? new_pp : new_qq) : a[0];
+    a[kK] = rotate ? 0.0 : a[kK];
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+template <int... kKs>
+__device__ __forceinline__ void parallel_sweep_double(double (&a)[16], double (&v)[16], int r, bool active,
+                                                      double threshold) {
+    (parallel_round_double<kKs>(a, v, r, active, threshold, std::make_integer_sequence<int, 16>{}), ...);
+}
+
+// fp64 re-solve of the flagged problems (Jacobi in double, the reference's
+// solver at its double instantiation, linalg.cpp:447-550: same rotation,
+// threshold 64 eps max(1, max|A|) with the double eps, stopping rule, ordering
+// and canonical vectors; the pairs in the parallel order), results rounded to
+// float.  Sixteen lanes per problem, four problems per wavefront at a time,
+// A and V in registers; the list length is read on the device, so no host
+// round trip is needed.  Bound by double-precision issue: the eight
+// rotations of a round share one divide and root chain.  Measured against
+// one problem per wavefront in the cyclic order with A and V in LDS: a
+// 501x283x6 YUV clip at rank 4, 443 us per half stage -> 76 us per stage.
 __global__ __launch_bounds__(64) void jacobi_refine_kernel(
     StageDesc d, int problem_stride, const int* __restrict__ problem_dims,
     const float* __restrict__ problems, const int* __restrict__ refine_list,
     const int* __restrict__ refine_count, float* __restrict__ eigenvalues,
     float* __restrict__ vectors, int* __restrict__ refined_total) {
     constexpr int kN = 16;
+    constexpr int kPerWave = 4;
     constexpr int kStride = kN + 1;
-    __shared__ double s_m[kN * kStride];
-    __shared__ double s_v[kN * kStride];
-    __shared__ int s_order[kN];
-    const int r = threadIdx.x;
+    __shared__ double s_v[kPerWave][kN * kStride];
+    __shared__ double s_diag[kPerWave][kN];
+    __shared__ int s_order[kPerWave][kN];
+    const int sub = threadIdx.x / kN;
+    const int r = threadIdx.x % kN;
     const int total = *refine_count;
-    if (blockIdx.x == 0 && r == 0 && refined_total != nullptr) {
+    if (blockIdx.x == 0 && threadIdx.x == 0 && refined_total != nullptr) {
         atomicAdd(refined_total, total);
     }
-    for (int item = blockIdx.x; item < total; item += gridDim.x) {
-        const int problem = refine_list[item];
-        const int group = problem / d.models;
-        const int n = problem_dims[group];
+    for (int first = blockIdx.x * kPerWave; first < total; first += gridDim.x * kPerWave) {
+        const bool valid = first + sub < total;
+        const int problem = refine_list[valid ? first + sub : first];
+        const int n = problem_dims[problem / d.models];
         const float* in = problems + static_cast<size_t>(problem) * problem_stride * problem_stride;
-        __syncthreads();
-        double row_max = 0.0;
-        if (r < kN) {
-            for (int c = 0; c < kN; ++c) {
-                double value = 0.0;
-                if (r < n && c < n) {
-                    value = static_cast<double>(in[r * problem_stride + c]);
-                    row_max = fmax(row_max, fabs(value));
-                }
-                s_m[r * kStride + c] = value;
-                s_v[r * kStride + c] = (r == c) ? 1.0 : 0.0;
+        double a[kN];
+        double v[kN];
+        double scale = 0.0;
+#pragma unroll
+        for (int j = 0; j < kN; ++j) {
+            const int col = r ^ j;
+            double value = 0.0;
+            if (r < n && col < n) {
+                value = static_cast<double>(in[r * problem_stride + col]);
+                scale = fmax(scale, fabs(value));
             }
+            a[j] = value;
+            v[j] = j == 0 ? 1.0 : 0.0;
         }
-        row_max = wave_max_double(row_max);
-        const double threshold = (64.0 * DBL_EPSILON) * (row_max > 1.0 ? row_max : 1.0);
-        __syncthreads();
+        const auto problem_max = [](double value) {
+            value = fmax(value, xor16<8>(value));
+            value = fmax(value, xor16<4>(value));
+            value = fmax(value, xor16<2>(value));
+            return fmax(value, xor16<1>(value));
+        };
+        scale = problem_max(scale);
+        const double threshold = (64.0 * DBL_EPSILON) * (scale > 1.0 ? scale : 1.0);
+        bool done = !valid || n <= 1;
+#pragma nounroll
         for (int sweep = 0; sweep < d.max_sweeps; ++sweep) {
             double off = 0.0;
-            if (r < n) {
-                for (int c = r + 1; c < n; ++c) {
-                    off = fmax(off, fabs(s_m[r * kStride + c]));
-                }
+#pragma unroll
+            for (int j = 1; j < kN; ++j) {
+                off = fmax(off, fabs(a[j]));
             }
-            off = wave_max_double(off);
-            if (off <= threshold) {
+            done = done || problem_max(off) <= threshold;
+            if (__all(done)) {
                 break;
             }
-            for (int p = 0; p + 1 < n; ++p) {
-                for (int q = p + 1; q < n; ++q) {
-                    const double apq = s_m[p * kStride + q];
-                    const bool rotate = fabs(apq) > threshold;  // uniform
-                    double c = 1.0;
-                    double sn = 0.0;
-                    double new_pp = 0.0;
-                    double new_qq = 0.0;
-                    double new_rp = 0.0;
-                    double new_rq = 0.0;
-                    double new_vp = 0.0;
-                    double new_vq = 0.0;
-                    if (rotate) {
-                        const double app = s_m[p * kStride + p];
-                        const double aqq = s_m[q * kStride + q];
-                        const double tau = (aqq - app) / (2.0 * apq);
-                        const double t_abs = 1.0 / (fabs(tau) + sqrt(1.0 + tau * tau));
-                        const double t = tau < 0.0 ? -t_abs : t_abs;
-                        c = 1.0 / sqrt(1.0 + t * t);
-                        sn = t * c;
-                        const double cc = c * c;
-                        const double ss = sn * sn;
-                        const double two_cs = 2.0 * (c * sn);
-                        new_pp = ((cc * app) - (two_cs * apq)) + (ss * aqq);
-                        new_qq = ((ss * app) + (two_cs * apq)) + (cc * aqq);
-                        if (r < n && r != p && r != q) {
-                            const double arp = s_m[r * kStride + p];
-                            const double arq = s_m[r * kStride + q];
-                            new_rp = (c * arp) - (sn * arq);
-                            new_rq = (sn * arp) + (c * arq);
-                        }
-                        if (r < n) {
-                            const double vrp = s_v[r * kStride + p];
-                            const double vrq = s_v[r * kStride + q];
-                            new_vp = (c * vrp) - (sn * vrq);
-                            new_vq = (sn * vrp) + (c * vrq);
-                        }
-                    }
-                    __syncthreads();
-                    if (rotate) {
-                        if (r < n && r != p && r != q) {
-                            s_m[r * kStride + p] = new_rp;
-                            s_m[p * kStride + r] = new_rp;
-                            s_m[r * kStride + q] = new_rq;
-                            s_m[q * kStride + r] = new_rq;
-                        }
-                        if (r == 0) {
-                            s_m[p * kStride + p] = new_pp;
-                            s_m[q * kStride + q] = new_qq;
-                            s_m[p * kStride + q] = 0.0;
-                            s_m[q * kStride + p] = 0.0;
-                        }
-                        if (r < n) {
-                            s_v[r * kStride + p] = new_vp;
-                            s_v[r * kStride + q] = new_vq;
-                        }
-                    }
-                    __syncthreads();
-                }
-            }
+            parallel_sweep_double<1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15>(a, v, r, !done, threshold);
         }
-        if (r < n) {
-            const double dr = s_m[r * kStride + r];
+        __syncthreads();  // the previous problems' vectors are written
+#pragma unroll
+        for (int j = 0; j < kN; ++j) {
+            s_v[sub][r * kStride + (r ^ j)] = v[j];
+        }
+        s_diag[sub][r] = a[0];
+        __syncthreads();
+        if (valid && r < n) {
+            const double dr = s_diag[sub][r];
             int rank = 0;
             for (int j = 0; j < n; ++j) {
-                const double dj = s_m[j * kStride + j];
+                const double dj = s_diag[sub][j];
                 rank += (dj > dr || (j < r && !(dr > dj))) ? 1 : 0;
             }
-            s_order[rank] = r;
+            s_order[sub][rank] = r;
         }
         __syncthreads();
-        if (r < d.rank && r < n) {
-            const int col = s_order[r];
+        if (valid && r < d.rank && r < n) {
+            const int col = s_order[sub][r];
+            const double* vs = s_v[sub];
             float* vec_out = vectors + (static_cast<size_t>(problem) * d.rank + r) * problem_stride;
             double norm_squared = 0.0;
             double max_abs = 0.0;
             int pivot = 0;
             for (int i = 0; i < n; ++i) {
-                const double value = s_v[i * kStride + col];
+                const double value = vs[i * kStride + col];
                 norm_squared += value * value;
                 if (fabs(value) > max_abs) {
                     max_abs = fabs(value);
                     pivot = i;
                 }
             }
-            double scale = 1.0;
+            double scale_out = 1.0;
             const bool rescale = norm_squared > DBL_MIN;
             if (rescale) {
-                scale = 1.0 / sqrt(norm_squared);
-                if (s_v[pivot * kStride + col] < 0.0) {
-                    scale = -scale;
+                scale_out = 1.0 / sqrt(norm_squared);
+                if (vs[pivot * kStride + col] < 0.0) {
+                    scale_out = -scale_out;
                 }
             }
             for (int i = 0; i < n; ++i) {
-                const double value = s_v[i * kStride + col];
-                vec_out[i] = static_cast<float>(rescale ? value * scale : value);
+                const double value = vs[i * kStride + col];
+                vec_out[i] = static_cast<float>(rescale ? value * scale_out : value);
             }
-            eigenvalues[static_cast<size_t>(problem) * d.rank + r] = static_cast<float>(s_m[col * kStride + col]);
+            eigenvalues[static_cast<size_t>(problem) * d.rank + r] = static_cast<float>(s_diag[sub][col]);
         }
     }
 }
