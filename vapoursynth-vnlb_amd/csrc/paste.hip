@@ -86,16 +86,22 @@ __device__ inline void for_each_clear(const StageDesc& d, const int* s_first, co
 // Clear targets of every anchor, computed in parallel (they do not depend
 // on the mask): a clear of a later anchor in the same 64-anchor chunk sets a
 // predecessor bit in that anchor's mask word; clears beyond the chunk are
-// listed.  Clears of earlier anchors cannot change any decision and are
-// dropped.
-__global__ __launch_bounds__(256) void paste_targets_kernel(
+// listed (in any order: clears commute).  Clears of earlier anchors cannot
+// change any decision and are dropped.  Sixteen lanes per anchor, one match
+// each: an anchor's matches are a chain of dependent lookups each, and a
+// thread walking 16 of them took 50 us for half of a 320x180x5 clip, this
+// takes 6 us (the walk below, with fewer scattered rows, 38 -> 24 us).
+constexpr int kTargetLanes = 16;
+constexpr int kTargetThreads = 256;
+__global__ __launch_bounds__(kTargetThreads) void paste_targets_kernel(
     StageDesc d, int frame_count, const int* __restrict__ frame_offsets,
     const int* __restrict__ frame_ids, const int* __restrict__ row_tables,
     const int* __restrict__ counts, const uint32_t* __restrict__ positions,
     unsigned long long* __restrict__ dep, int* __restrict__ target_counts,
     int* __restrict__ targets, int target_stride) {
     // frame_offsets are clip-wide anchor indices; the range may start past 0.
-    const int a = frame_offsets[0] + blockIdx.x * blockDim.x + threadIdx.x;
+    const int lane = threadIdx.x % kTargetLanes;
+    const int a = frame_offsets[0] + blockIdx.x * (kTargetThreads / kTargetLanes) + threadIdx.x / kTargetLanes;
     const int total = frame_offsets[frame_count];
     if (a >= total) {
         return;
@@ -117,22 +123,51 @@ __global__ __launch_bounds__(256) void paste_targets_kernel(
     const uint32_t* list = positions + static_cast<size_t>(a) * d.cap;
     int* out = targets + static_cast<size_t>(a) * target_stride;
     int n = 0;
-    for (int k = 0; k < similar; ++k) {
-        for_each_clear(d, r_first, r_phase, r_count, list[k], anchor_frame, [&](int t) {
-            if (t <= local) {
-                return;
+    for (int k0 = 0; k0 < similar; k0 += kTargetLanes) {
+        int found[5];
+        int mine = 0;
+#pragma unroll
+        for (int i = 0; i < 5; ++i) {
+            found[i] = -1;
+        }
+        if (k0 + lane < similar) {
+            int i = 0;
+            for_each_clear(d, r_first, r_phase, r_count, list[k0 + lane], anchor_frame, [&](int t) {
+                if (t > local && t < chunk_end) {
+                    atomicOr(&dep[first + t], 1ull << (local & 63));
+                } else if (t > local) {
+#pragma unroll
+                    for (int j = 0; j < 5; ++j) {
+                        found[j] = j == i ? t : found[j];
+                    }
+                    ++mine;
+                }
+                ++i;
+            });
+        }
+        // Places of the lane's targets after those of the lanes before it.
+        int before = mine;
+#pragma unroll
+        for (int offset = 1; offset < kTargetLanes; offset <<= 1) {
+            const int other = __shfl_up(before, offset, kTargetLanes);
+            before += lane >= offset ? other : 0;
+        }
+        const int all = __shfl(before, kTargetLanes - 1, kTargetLanes);
+        int at = n + before - mine;
+#pragma unroll
+        for (int i = 0; i < 5; ++i) {
+            if (found[i] >= 0 && at < target_stride) {
+                out[at++] = found[i];
             }
-            if (t < chunk_end) {
-                atomicOr(&dep[first + t], 1ull << (local & 63));
-            } else if (n < target_stride) {
-                out[n++] = t;
-            }
-        });
+        }
+        n = min(n + all, target_stride);
     }
     // An anchor without matches (every candidate distance NaN) is not a
     // group and clears nothing (process_anchor_impl skips it,
     // core.cpp:1851-1903): marked with a negative target count.
-    target_counts[a] = similar > 0 ? n : -1;
+    if (lane == 0) {
+        target_counts[a] = similar > 0 ? n : -1;
+    }
 }
 
 // The serial raster walk, 64 anchors at a time: wave-wide rounds over the
@@ -303,8 +338,10 @@ hipError_t launch_paste(const StageDesc& d, int frame_count, const int* frame_of
         return hipSuccess;
     }
     const int stride = paste_target_stride(d);
-    hipLaunchKernelGGL(paste_targets_kernel, dim3(static_cast<unsigned>((anchor_count + 255) / 256)),
-                       dim3(256), 0, stream, d, frame_count, frame_offsets, frame_ids, row_tables,
+    constexpr int kAnchorsPerBlock = kTargetThreads / kTargetLanes;
+    hipLaunchKernelGGL(paste_targets_kernel,
+                       dim3(static_cast<unsigned>((anchor_count + kAnchorsPerBlock - 1) / kAnchorsPerBlock)),
+                       dim3(kTargetThreads), 0, stream, d, frame_count, frame_offsets, frame_ids, row_tables,
                        counts, positions, dep, target_counts, targets, stride);
     hipError_t status = hipGetLastError();
     if (status != hipSuccess) {

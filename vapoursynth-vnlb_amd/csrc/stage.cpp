@@ -1027,6 +1027,18 @@ void run_stage(vnlbhip_context& ctx, int stage, const vnlbhip_params& p, const f
         unsigned long long* d_dep = ctx.paste_dep.reserve(anchor_count);
         int* d_tcount = ctx.paste_target_counts.reserve(anchor_count);
         int* d_targets = ctx.paste_targets.reserve(vnlbhip::paste_targets_size(d, anchor_count));
+        if (lists != nullptr) {
+            // The lists go out whole: entries past an anchor's count are zero
+            // instead of what the buffers last held.
+            untimed(ctx, "clear positions", [&]() {
+                return vnlbhip::launch_fill_zero_int(reinterpret_cast<int*>(d_positions),
+                                                     static_cast<size_t>(anchor_count) * cap, stream);
+            });
+            untimed(ctx, "clear distances", [&]() {
+                return vnlbhip::launch_fill_zero_int(reinterpret_cast<int*>(d_distances),
+                                                     static_cast<size_t>(anchor_count) * cap, stream);
+            });
+        }
         untimed(ctx, "clear paste masks", [&]() { return vnlbhip::launch_fill_zero(reinterpret_cast<double*>(d_dep), anchor_count, stream); });
         untimed(ctx, "clear group counts", [&]() { return vnlbhip::launch_fill_zero_int(d_group_count, kMaxParts, stream); });
 
