@@ -1093,9 +1093,11 @@ hipError_t launch_jacobi(const StageDesc& d, const int* group_count_dev, int pro
     if (n > 128) {
         return hipErrorInvalidValue;
     }
-    // Up to 16 rows a problem fits the registers of four lanes (512 of the
-    // lane's 512 registers would hold 20 rows); above, one or two problems per
-    // wavefront with A in LDS.
+    // Up to 16 rows the wavefront's rotations are bound by issue, and four
+    // lanes per problem share them among 16 problems (128 registers of A and
+    // V a lane at 16 rows; 32 rows would take 512): see the figures at
+    // jacobi_quad_kernel.  Above, one or two problems per wavefront with A in
+    // LDS (figures at jacobi_wave_kernel's comment).
     const size_t shared = jacobi_problem_floats(n) * sizeof(float);
     if (n <= 4) {
         VNLBHIP_JACOBI(jacobi_quad_kernel<1>, 16, 0);
