@@ -85,8 +85,8 @@ __device__ inline void rotate_pair(const Rotation& o, float& left, float& right)
     right = (o.s * l) + (o.c * r);
 }
 
-// The kRank-th eigenpair from V (rows of `stride` floats in LDS) and the
-// diagonal: the canonical vector of column col, read in row order.
+// The canonical vector of column col of V (rows of `stride` floats in LDS),
+// read in row order.
 __device__ inline void write_eigenvector(const float* __restrict__ v, int stride, int n, int col,
                                          float* __restrict__ out) {
     float norm_squared = 0.0F;
