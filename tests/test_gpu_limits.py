@@ -152,3 +152,15 @@ def test_jacobi_sweep_limit_and_unconverged_problems(oracle_lib):
             ctx.set_jacobi(0)
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("patch_time,radius", [(145, 63), (146, 63), (242, 14), (256, 0)])
+def test_long_patches_of_small_blocks(gpu, oracle_lib, patch_time, radius):
+    """2x2 patches of many frames in 9x9 windows, the shapes whose 16-byte rows
+    exceed the matcher's LDS unguided (all but the first): match lists and
+    eigenvalues bit for bit."""
+    noisy, _ = synth.make_clip(14, 12, 256, 1, sigma8=20, seed=patch_time, motion="subpixel")
+    bp = parse_stage_parameters(BASIC, dict(sigma=20, block_size=2, block_step=3, group_size=8, bm_range=4,
+                                            patch_time=patch_time, search_bwd=0, search_fwd=radius, rank=4, tau=0))
+    print(f"[limits] {patch_time} patch frames, {radius} following frames", flush=True)
+    _compare_frame(gpu, oracle_lib, BASIC, bp, noisy, None, 0)

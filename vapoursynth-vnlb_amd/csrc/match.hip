@@ -12,6 +12,7 @@
 #include "common.h"
 #include "device_util.h"
 #include "kernels.h"
+#include "match_layout.h"
 #include "proposer.h"
 #include "select.h"
 
@@ -19,8 +20,6 @@
 
 namespace vnlbhip {
 namespace {
-
-constexpr int kMatchThreads = 256;
 
 // Row distance of 4 horizontally adjacent candidates (values[j ..]) against
 // one reference row, each added to its running distance in the reference's
@@ -121,41 +120,6 @@ struct Region {
     int floats;    // frames * rows * cols (+ padding)
 };
 
-// Unguided: the scheduled frames share one window, frames t_low ..
-// t_high + Pt - 1.  Guided: every scheduled frame has its own window, so
-// each (frame, patch frame) pair has its own plane.
-__host__ __device__ inline int region_floats(int window, int patch, int temporal, int patch_time,
-                                             bool guided) {
-    const int side = window + patch - 1;
-    return (guided ? temporal * patch_time : temporal + patch_time - 1) * side * side + 8;
-}
-
-// The exhaustive matcher's region: rows of a 16-byte multiple that hold the
-// four samples past the last group of four candidates, and one row more (the
-// second of a pair of candidate rows may lie past the window).  Where that
-// exceeds the LDS of a workgroup, rows as narrow as region_floats has them.
-__host__ __device__ inline int region_pitch(int window, int patch, bool wide) {
-    return wide ? (window + 3) / 4 * 4 + (patch + 3 + 3) / 4 * 4 - 4 : window + patch - 1;
-}
-__host__ __device__ inline int match_region_floats(int window, int patch, int temporal, int patch_time, bool guided,
-                                                   bool wide) {
-    const int rows = (guided ? temporal * patch_time : temporal + patch_time - 1) * (window + patch - 1);
-    return wide ? ((rows + 1) * region_pitch(window, patch, true) + 3) / 4 * 4
-                : region_floats(window, patch, temporal, patch_time, guided) + window + patch - 1;
-}
-
-// Candidate distances of a full window: window^2 per scheduled frame.
-__host__ __device__ inline int window_candidates(const StageDesc& d) {
-    return d.search_window * d.search_window * (d.search_bwd + d.search_fwd + 1);
-}
-
-// Entries of each of the three selection arrays after the distances: the
-// selected list (at most the cap) and the short path's candidate list (at
-// most one per thread).
-__host__ __device__ inline int selection_entries(const StageDesc& d) {
-    return d.cap > kMatchThreads ? d.cap : kMatchThreads;
-}
-
 // Distances (scan order) with the search region staged in LDS one channel
 // at a time; each thread owns 4 horizontally adjacent candidates of one row,
 // or of two where one row each would fill the workgroup more than once, so
@@ -247,14 +211,13 @@ __global__ __launch_bounds__(kMatchThreads) void match_kernel(
     const int pitch = region_pitch(d.search_window, P, kWide);
     const int plane = rrows * pitch;
 
+    const MatchLayout L = match_layout(d, P, guided, kWide);
     float* s_region = s_dyn;
-    float* s_dist = s_dyn + match_region_floats(d.search_window, P, d.search_bwd + d.search_fwd + 1,
-                                                d.patch_time, guided, kWide);
-    // Selection scratch after the candidate distances.
-    float* s_sel_dist = s_dist + window_candidates(d);
+    float* s_dist = s_dyn + L.dist;
+    float* s_sel_dist = s_dyn + L.sel;
     int* s_sel_index = reinterpret_cast<int*>(s_sel_dist + selection_entries(d));
     int* s_sel_rank = s_sel_index + selection_entries(d);
-    float* s_ref = reinterpret_cast<float*>(s_sel_rank + selection_entries(d));
+    float* s_ref = s_dyn + L.ref;
 
     const int groups_x = (nx + 3) >> 2;
     const bool paired = nt * ny * groups_x > kMatchThreads;
@@ -759,33 +722,28 @@ hipError_t launch_match(const StageDesc& d, const float* source,
     const dim3 grid(static_cast<unsigned>(anchor_count));
     const dim3 block(kMatchThreads);
     const bool guided = offsets != nullptr;
-    const int temporal = d.search_bwd + d.search_fwd + 1;
-    // Guided windows have a plane per scheduled and patch frame; wide rows may
-    // not fit beside them (unguided ones always do: at most 108 KB narrow).
-    const size_t others = match_shared_bytes(d, guided) -
-                          sizeof(float) * region_floats(d.search_window, d.patch, temporal, d.patch_time, guided);
-    const auto shared_bytes = [&](bool wide) {
-        return others + sizeof(float) * match_region_floats(d.search_window, d.patch, temporal, d.patch_time,
-                                                            guided, wide) +
-               sizeof(float) * d.dim;
-    };
-    constexpr size_t kMatchLds = 156 * 1024;  // 160 KB less the kernel's static arrays
-    const bool wide = shared_bytes(true) <= kMatchLds;
-    const size_t shared = shared_bytes(wide);
+    const bool wide = match_wide_rows(d, guided);
+    const size_t shared = match_layout(d, d.patch, guided, wide).words * sizeof(float);
 #define VNLBHIP_MATCH(PV, GUIDED, WIDE)                                                          \
     hipLaunchKernelGGL((match_kernel<PV, GUIDED, WIDE>), grid, block, shared, stream, d, source, \
                        anchors, anchor_count, counts, positions, distances, offsets,             \
                        offsets_temporal)
     switch (d.patch) {
-#define VNLBHIP_MATCH_CASE(PV)                  \
-    case PV:                                    \
-        if (!guided) {                          \
-            VNLBHIP_MATCH(PV, false, true);     \
-        } else if (wide) {                      \
-            VNLBHIP_MATCH(PV, true, true);      \
-        } else {                                \
-            VNLBHIP_MATCH(PV, true, false);     \
-        }                                       \
+#define VNLBHIP_MATCH_CASE(PV)                                       \
+    case PV:                                                         \
+        if (wide) {                                                  \
+            if (guided) {                                            \
+                VNLBHIP_MATCH(PV, true, true);                       \
+            } else {                                                 \
+                VNLBHIP_MATCH(PV, false, true);                      \
+            }                                                        \
+        } else if (guided) {                                         \
+            VNLBHIP_MATCH(PV, true, false);                          \
+        } else if constexpr (narrow_unguided_patch(PV)) {            \
+            VNLBHIP_MATCH(PV, false, false);                         \
+        } else {                                                     \
+            return hipErrorInvalidValue;  /* past kMatchBudget */    \
+        }                                                            \
         break;
         VNLBHIP_MATCH_CASE(1)
         VNLBHIP_MATCH_CASE(2)
