@@ -1,5 +1,6 @@
 """LDS layout of the exhaustive matcher, on the CPU: every shape that it is
 launched for fits its allocation and has a kernel (match_layout_check.cpp)."""
+import re
 import subprocess
 from pathlib import Path
 
@@ -15,3 +16,17 @@ def test_every_shape_fits_its_allocation(tmp_path):
     assert run.returncode == 0, run.stdout
     # Unguided narrow rows: 2x2 patches only, and some of them.
     assert [line.split(":")[0] for line in run.stdout.splitlines() if line.startswith("unguided")] == ["unguided 2"]
+
+
+def test_dynamic_lds_is_aligned_for_vector_reads(tmp_path):
+    """The dynamic LDS array of every kernel in the file starts at a multiple
+    of 16 bytes by its type, not by what the static arrays before it add up to
+    (the learned matcher's s_dyn is read a float at a time)."""
+    import build as hip_build  # vapoursynth-vnlb_amd/build.py
+
+    ir = tmp_path / "match.ll"
+    subprocess.run([hip_build.hipcc(), *hip_build.COMMON_FLAGS, "--cuda-device-only", "-emit-llvm", "-S", "-Xclang",
+                    "-disable-llvm-passes", str(CSRC / "match.hip"), "-o", str(ir)], check=True, capture_output=True)
+    arrays = re.findall(r"^@(\S+) = external addrspace\(3\) global .*, align (\d+)$", ir.read_text(), re.M)
+    aligned = {name: int(align) for name, align in arrays if "s_dyn" not in name}
+    assert len(aligned) == 1 and min(aligned.values()) >= 16, arrays

@@ -136,7 +136,8 @@ __global__ __launch_bounds__(kMatchThreads) void match_kernel(
     StageDesc d, const float* __restrict__ source, const uint32_t* __restrict__ anchors,
     int anchor_count, int* __restrict__ counts, uint32_t* __restrict__ positions,
     float* __restrict__ distances, const int16_t* __restrict__ offsets, int offsets_temporal) {
-    extern __shared__ float s_dyn[];
+    extern __shared__ float4 s_match4[];  // (rows are read 16 bytes at a time)
+    float* s_dyn = reinterpret_cast<float*>(s_match4);
     // Guided search: the window origin of each scheduled frame.
     __shared__ int s_frame_x_low[kMaxTemporal];
     __shared__ int s_frame_y_low[kMaxTemporal];
