@@ -96,6 +96,10 @@ __device__ inline void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Device memory: a pointer made from an integer is a FLAT one otherwise, whose
+// loads count with the LDS accesses and are waited for with them.
+using GlobalFloat = __attribute__((address_space(1))) float;
+
 // v of lane j (uniform).
 __device__ inline float lane_value(float v, int j) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), j));
@@ -682,7 +686,7 @@ __global__ __launch_bounds__(kModelThreads, 3) void filter_fast_kernel(
                 for (int s2 = 0; s2 < kFastModel; ++s2) {
                     const uint64_t lo = static_cast<uint32_t>(__builtin_amdgcn_readlane(row_lo, s2));
                     const uint64_t hi = static_cast<uint32_t>(__builtin_amdgcn_readlane(row_hi, s2));
-                    const float* row = reinterpret_cast<const float*>(hi << 32 | lo);
+                    const GlobalFloat* row = reinterpret_cast<const GlobalFloat*>(hi << 32 | lo);
 #pragma unroll
                     for (int tt = 0; tt < kPt; ++tt) {
                         x[tt][s2] = row[in_off[tt]];
