@@ -18,7 +18,7 @@ def _disassembly(source, tmp_path):
     return subprocess.run([f"{LLVM}/llvm-objdump", "-d", str(code)], check=True, capture_output=True, text=True).stdout
 
 
-@pytest.mark.parametrize("source", ["filter_fast.hip"])
+@pytest.mark.parametrize("source", ["filter.hip", "filter_fast.hip"])
 def test_no_flat_memory_instructions(source, tmp_path):
     """Kernels read and write device memory and LDS by instructions of their
     own.  A FLAT access counts as both, so every wait for the LDS waits for

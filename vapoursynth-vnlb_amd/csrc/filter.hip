@@ -312,6 +312,17 @@ __device__ __forceinline__ void plan_boxes(const StageDesc& d, const uint32_t* _
     }
 }
 
+// Sums in LDS and in device memory, by the pointer's type: through plain
+// pointers the compiler joins the two into FLAT atomics.
+using LdsDouble = __attribute__((address_space(3))) double;
+using GlobalDouble = __attribute__((address_space(1))) double;
+__device__ inline void add_double(LdsDouble* p, double v) {
+    __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ inline void add_double(GlobalDouble* p, double v) {
+    __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // One round of samples (one per team, position p, weight w, the filtered row
 // of model m in `out`; teams without a sample have held false) into the
 // accumulators, through the tile.  Slots 4 q + i of a row are the 64 pixels
@@ -339,14 +350,14 @@ __device__ __forceinline__ void aggregate_tile(const StageDesc& d, double* __res
     const size_t plane = static_cast<size_t>(d.height) * d.width;
     // Adds the sample's pixels of patch time t: value plane by value plane
     // from `cell` (plane_step apart), the weights into `weight`.
-    const auto add = [&](int t, double* cell, size_t plane_step, int row_step, double* weight) {
+    const auto add = [&](int t, auto* cell, size_t plane_step, int row_step, auto* weight) {
         int next = t;
 #pragma unroll
         for (int q = 0; q < kS / 4; ++q) {
             if (q == next) {  // uniform
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    unsafeAtomicAdd(cell + 2 * i * row_step, static_cast<double>(cw[i] * pinned(out[4 * q + i])));
+                    add_double(cell + 2 * i * row_step, static_cast<double>(cw[i] * pinned(out[4 * q + i])));
                 }
                 cell += plane_step;
                 next += d.patch_time;
@@ -355,7 +366,7 @@ __device__ __forceinline__ void aggregate_tile(const StageDesc& d, double* __res
         if (m == 0) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                unsafeAtomicAdd(weight + 2 * i * row_step, static_cast<double>(cw[i]));
+                add_double(weight + 2 * i * row_step, static_cast<double>(cw[i]));
             }
         }
     };
@@ -367,12 +378,13 @@ __device__ __forceinline__ void aggregate_tile(const StageDesc& d, double* __res
             if (held && slot >= 0 && slot < d.slots) {
                 const TileBox box = boxes[slot];
                 if (box.batch == batch) {
-                    double* cell = tile + box.cell + (py - box.y0) * box.width + px - box.x0;
+                    LdsDouble* cell = (LdsDouble*)tile + box.cell + (py - box.y0) * box.width + px - box.x0;
                     add(t, cell, cells, box.width, cell + channels * cells);
                 } else if (batch == 0 && box.batch < 0) {
                     // Boxes too large for the tile.
-                    double* frame = acc + static_cast<size_t>(af + slot - d.search_bwd) * (d.channels + 1) * plane +
-                                    static_cast<size_t>(py) * d.width + px;
+                    GlobalDouble* frame = (GlobalDouble*)acc +
+                                          static_cast<size_t>(af + slot - d.search_bwd) * (d.channels + 1) * plane +
+                                          static_cast<size_t>(py) * d.width + px;
                     add(t, frame + c_first * plane, plane, d.width, frame + d.channels * plane);
                 }
             }
