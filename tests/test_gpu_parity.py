@@ -161,6 +161,25 @@ def test_nan_region_anchors_are_skipped(gpu, oracle_lib):
     assert np.abs(got[finite] - want[finite]).max() <= MAX_ABS
 
 
+@pytest.mark.parametrize("group_size,patch_time", [(3, 2), (12, 2), (24, 2), (40, 2), (70, 1)])
+def test_infinite_sample_in_the_models(gpu, oracle_lib, group_size, patch_time):
+    """An infinite chroma sample, which Basic does not match on, leaves models
+    with infinite and NaN diagonals: every eigenpair still has a place, and
+    the output is the oracle's (its tolerance above, the sample itself
+    aside) at each of the solver's sizes."""
+    noisy, _ = synth.make_clip(48, 40, 4, 3, sigma8=15, seed=31, motion="subpixel")
+    noisy = noisy.copy()
+    noisy[1, 1, 20, 24] = np.inf
+    p = parse_stage_parameters(BASIC, dict(sigma=15, block_size=8, block_step=4, group_size=group_size, bm_range=5,
+                                           patch_time=patch_time, radius=1, rank=min(group_size, 8), tau=0, chroma=1))
+    print(f"[inf] {group_size} neighbours", flush=True)
+    want, _ = oracle_lib.stage(BASIC, p, noisy, flags=oracle_lib.ACCUM_DOUBLE)
+    got = gpu.stage(BASIC, p, _dev(noisy)).cpu().numpy().reshape(want.shape)
+    np.testing.assert_array_equal(np.isfinite(got), np.isfinite(want))
+    finite = np.isfinite(want)
+    assert np.abs(got[finite] - want[finite]).max() <= MAX_ABS
+
+
 def test_constant_clip(gpu):
     noisy = np.full((3, 1, 24, 20), 0.25, np.float32)
     p = StageParameters(sigma=0.1, patch_size=2, patch_time=1, search_window=3, search_bwd=1,

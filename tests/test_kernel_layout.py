@@ -1,5 +1,6 @@
-"""LDS layout of the exhaustive matcher, on the CPU: every shape that it is
-launched for fits its allocation and has a kernel (match_layout_check.cpp)."""
+"""Host checks of what the kernels and their launches share, on the CPU: the
+exhaustive matcher's LDS layout (every shape that it is launched for fits its
+allocation and has a kernel) and the order of eigenpairs."""
 import re
 import subprocess
 from pathlib import Path
@@ -8,14 +9,23 @@ TESTS = Path(__file__).resolve().parent
 CSRC = TESTS.parent / "vapoursynth-vnlb_amd" / "csrc"
 
 
-def test_every_shape_fits_its_allocation(tmp_path):
-    program = tmp_path / "match_layout_check"
+def _run(name, tmp_path):
+    program = tmp_path / name
     subprocess.run(["g++", "-O2", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", f"-I{CSRC}",
-                    str(TESTS / "match_layout_check.cpp"), "-o", str(program)], check=True)
+                    str(TESTS / f"{name}.cpp"), "-o", str(program)], check=True)
     run = subprocess.run([str(program)], capture_output=True, text=True)
     assert run.returncode == 0, run.stdout
+    return run.stdout
+
+
+def test_every_match_shape_fits_its_allocation(tmp_path):
+    out = _run("match_layout_check", tmp_path)
     # Unguided narrow rows: 2x2 patches only, and some of them.
-    assert [line.split(":")[0] for line in run.stdout.splitlines() if line.startswith("unguided")] == ["unguided 2"]
+    assert [line.split(":")[0] for line in out.splitlines() if line.startswith("unguided")] == ["unguided 2"]
+
+
+def test_eigenpair_places_are_a_permutation(tmp_path):
+    _run("eigen_order_check", tmp_path)
 
 
 def test_dynamic_lds_is_aligned_for_vector_reads(tmp_path):

@@ -6,6 +6,7 @@
 // 16-lane summation order of the CPU restatement.
 #include "common.h"
 #include "device_util.h"
+#include "eigen_order.h"
 #include "group.h"
 #include "kernels.h"
 
@@ -214,13 +215,13 @@ __device__ __forceinline__ void quad_sweep(float (&a)[kSlots][4 * kSlots], float
 // problems would halve the wavefronts per compute unit.
 template <int kSlots, int kC, int... kI>
 __device__ __forceinline__ void quad_output_column(const float (&v)[kSlots][4 * kSlots],
-                                                   const float (&diag)[4 * kSlots], int l,
-                                                   bool valid, int n, int rank_limit, int stride,
+                                                   const float (&diag)[4 * kSlots],
+                                                   const float (&keys)[4 * kSlots], int l, bool valid, int n, int rank_limit, int stride,
                                                    float* __restrict__ vectors, float* __restrict__ values,
                                                    std::integer_sequence<int, kI...>) {
     const float dr = diag[kC];
     int rank = 0;
-    ((rank += kI < n && (diag[kI] > dr || (kI < kC && !(dr > diag[kI]))) ? 1 : 0), ...);
+    ((rank += kI < n && kI != kC && ordered_before(keys[kI], keys[kC], kI < kC) ? 1 : 0), ...);
     float norm_squared = 0.0F;
     float max_abs = 0.0F;
     float pivot = quad_lane<0>(v[0][kC]);
@@ -263,7 +264,8 @@ __device__ __forceinline__ void quad_output(const float (&a)[kSlots][4 * kSlots]
                                             int rank_limit, int stride, float* __restrict__ vectors,
                                             float* __restrict__ values, std::integer_sequence<int, kI...> all) {
     const float diag[] = {quad_lane<kI % 4>(a[kI / 4][kI])...};
-    (quad_output_column<kSlots, kI>(v, diag, l, valid, n, rank_limit, stride, vectors, values, all), ...);
+    const float keys[] = {order_key(diag[kI])...};
+    (quad_output_column<kSlots, kI>(v, diag, keys, l, valid, n, rank_limit, stride, vectors, values, all), ...);
 }
 
 template <int kSlots>
@@ -620,13 +622,7 @@ __global__ __launch_bounds__(64) void jacobi_wave_kernel(
     }
     __syncthreads();
     for (int r = lane; valid && r < n; r += kLP) {
-        const float dr = diagonal[r];
-        int rank = 0;
-        for (int j = 0; j < n; ++j) {
-            const float dj = diagonal[j];
-            rank += (dj > dr || (j < r && !(dr > dj))) ? 1 : 0;
-        }
-        order[rank] = r;
+        order[descending_place(diagonal, n, r)] = r;
     }
     __syncthreads();
     const bool writes = valid && lane < d.rank && lane < n;
@@ -847,13 +843,7 @@ __global__ __launch_bounds__(64) void jacobi_parallel_kernel(
     s_diag[sub][r] = a[0];
     __syncthreads();
     if (valid && r < n) {
-        const float dr = s_diag[sub][r];
-        int rank = 0;
-        for (int j = 0; j < n; ++j) {
-            const float dj = s_diag[sub][j];
-            rank += (dj > dr || (j < r && !(dr > dj))) ? 1 : 0;
-        }
-        s_order[sub][rank] = r;
+        s_order[sub][descending_place(s_diag[sub], n, r)] = r;
     }
     __syncthreads();
     if (valid && r < d.rank && r < n) {
@@ -1035,13 +1025,7 @@ __global__ __launch_bounds__(64) void jacobi_refine_kernel(
         s_diag[sub][r] = a[0];
         __syncthreads();
         if (valid && r < n) {
-            const double dr = s_diag[sub][r];
-            int rank = 0;
-            for (int j = 0; j < n; ++j) {
-                const double dj = s_diag[sub][j];
-                rank += (dj > dr || (j < r && !(dr > dj))) ? 1 : 0;
-            }
-            s_order[sub][rank] = r;
+            s_order[sub][descending_place(s_diag[sub], n, r)] = r;
         }
         __syncthreads();
         if (valid && r < d.rank && r < n) {
