@@ -46,8 +46,7 @@ struct Rotation {
 
 // Square root and reciprocal of x >= 1, correctly rounded: the hardware's
 // approximation and one Newton step on its residual.  Compared with sqrtf
-// and 1.0F / x for every float in [1, 2^32): no difference (both depend on
-// the mantissa and, for the root, the exponent's parity alone).  Without the
+// and 1.0F / x for every float in [1, 2^52): no difference.  Without the
 // general case's scaling and special values they are 4 and 3 dependent
 // instructions instead of 15 and 11.
 __device__ __forceinline__ float sqrt_from_one(float x) {
@@ -60,9 +59,10 @@ __device__ __forceinline__ float reciprocal_from_one(float x) {
     return fmaf(fmaf(-x, r, 1.0F), r, r);
 }
 
-// A rotating pivot is above 64 float epsilons of max |A| and the diagonal at
-// most n max |A| = 128 max |A|, so |tau| is below 2^25 and the two roots and
-// reciprocals stay within the range above.
+// A rotating pivot is above 64 float epsilons (2^-17) of max |A| and the
+// diagonal at most n max |A| = 128 max |A| in magnitude, so |tau| is at most
+// 2^24: the first root's argument is at most 1 + 2^48, its reciprocal's 2^25
+// and the second pair's 2, all within the range compared above.
 __device__ __forceinline__ Rotation rotation_of(float app, float aqq, float apq) {
     Rotation o;
     const float tau = (aqq - app) / (2.0F * apq);
@@ -746,7 +746,7 @@ __device__ inline void parallel_sweep(float (&a)[16], float (&v)[16], int r, boo
     (parallel_round<kKs>(a, v, r, active, threshold), ...);
 }
 
-// Same sweep structure and canonical vectors as jacobi_kernel, with the
+// Same sweep structure and canonical vectors as the cyclic kernels above, with the
 // parallel ordering above: 16 lanes per problem, four per wavefront.  The
 // sweeps stop once every off-diagonal entry is at most 2^-14 of
 // max(1, max |A|) (the exact form stops at 64 float epsilons, about 2^-17):
