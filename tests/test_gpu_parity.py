@@ -11,6 +11,7 @@ import numpy as np
 import pytest
 import torch
 
+import vnlbhip
 import workloads
 from vnlbhip import synth
 from vnlbhip.params import BASIC, FINAL, StageParameters, parse_stage_parameters
@@ -252,3 +253,32 @@ def test_aggregation_paths(gpu, oracle_lib, channels, extra):
     final = gpu.stage(FINAL, fp, _dev(noisy), _dev(want_basic))
     for got, want in ((basic, want_basic), (final, want_final)):
         assert np.abs(got.cpu().numpy().reshape(want.shape) - want).max() <= 5e-6
+
+
+@pytest.mark.parametrize("form", ["plain", "fast"])
+@pytest.mark.parametrize("width,height,frames,extra", [
+    # 81 k anchors: past the joined lists of small batches.
+    (138, 131, 5, dict(block_size=8, block_step=1, group_size=8, rank=8, bm_range=2)),
+    # 22 k anchors of 112-row models: past their bytes.
+    (76, 72, 6, dict(block_size=8, block_step=1, group_size=112, rank=8, bm_range=5, patch_time=2))])
+def test_batches_of_separate_group_lists(oracle_lib, form, width, height, frames, extra):
+    """Batches whose parts keep their group lists and model launches: the
+    oracle's groups; outputs within the plain form's tolerance, 0.05 dB in
+    the fast one."""
+    noisy, clean = synth.make_clip(width, height, frames, 1, sigma8=15, seed=77, motion="subpixel")
+    p = parse_stage_parameters(BASIC, dict(dict(sigma=15, radius=1, tau=0, patch_time=1), **extra))
+    print(f"[parity] separate lists, {form}, {width}x{height}x{frames}", flush=True)
+    ctx = vnlbhip.Context(0)
+    try:
+        ctx.set_form(form)
+        got = ctx.stage(BASIC, p, _dev(noisy)).cpu().numpy()
+        stats = ctx.stats()
+    finally:
+        ctx.close()
+    want, groups = oracle_lib.stage(BASIC, p, noisy, flags=oracle_lib.ACCUM_DOUBLE, threads=4)
+    assert stats["parts"] > 1
+    if form == "plain":
+        assert stats["groups"] == groups
+        _check_output(got.reshape(want.shape), want, clean)
+    else:
+        assert abs(synth.psnr(got.reshape(want.shape), clean) - synth.psnr(want, clean)) <= 0.05

@@ -539,8 +539,14 @@ constexpr int kDefaultParts = 2;
 // (256x256x5 GrayS, 5.4 k anchors: 1134 us a pass with two model launches per
 // stage, 940 us with one; 717x403x7 uncoupled YUV, 57 k anchors: 9.79 ->
 // 9.56 ms).  Above, the first part's model covers the last part's paste scan
-// (150 k anchors: 16.1 ms against 16.2 without).
+// (150 k anchors: 16.1 ms against 16.2 without).  Larger models gain as well
+// (Basic on grey clips, two launches -> one: 3.7 k anchors, 24 rows 2.10 ->
+// 1.30 ms, 64 rows 10.7 -> 6.6 ms; 61 k anchors, 24 rows 9.80 -> 9.24 ms, 64
+// rows 76.1 -> 72.9 ms, 100 rows 393 -> 381 ms), but a joined list's model
+// buffers hold the whole batch instead of a part: past kJoinedFloats (1 GiB)
+// the lists stay separate, which bounds what joining adds at half of that.
 constexpr int kJoinedAnchors = 1 << 16;
+constexpr size_t kJoinedFloats = static_cast<size_t>(1) << 28;
 
 struct vnlbhip_context {
     int device = 0;
@@ -1055,7 +1061,11 @@ void run_stage(vnlbhip_context& ctx, int stage, const vnlbhip_params& p, const f
             part_frame[h] = frame_count * h / parts;
         }
         // (A scratch call keeps the smaller buffers of separate lists.)
-        const bool joined = anchor_count <= kJoinedAnchors && !ctx.generation.arena.active;
+        // Eigen problems, eigenvectors and means of a group.
+        const size_t group_floats = static_cast<size_t>(d.models) * n_stride * (n_stride + d.rank) + 2 * d.dim;
+        const bool joined = anchor_count <= kJoinedAnchors &&
+                            static_cast<size_t>(anchor_count) * group_floats <= kJoinedFloats &&
+                            !ctx.generation.arena.active;
         check(hipEventRecord(ctx.ready_event, stream), "hipEventRecord");
         check(hipStreamWaitEvent(ctx.side, ctx.ready_event, 0), "hipStreamWaitEvent");
 
