@@ -16,8 +16,6 @@
 #include "proposer.h"
 #include "select.h"
 
-#include <type_traits>
-
 namespace vnlbhip {
 namespace {
 
@@ -130,8 +128,12 @@ struct Region {
 // instructions of a wavefront) with the LDS reads beside them: sharing a row
 // between two candidate rows, 16-byte reads, the reference patch from scalar
 // loads and the staging by rows took 201 k anchors of a 1280x720 YUV clip
-// (mean of both stages) from 8.6 to 7.3 ms.
-template <int kP, bool kGuided, bool kWide>
+// (mean of both stages) from 8.6 to 7.3 ms.  Windows of one row per thread
+// (kRows = 1) have kernels of their own, with the reference patch in LDS at a
+// 16-byte address and a sample per thread staged: in the kernel of two rows
+// they paid for its registers and its batches (8x8 patches, 5x5x3 windows of a
+// 200x150x4 grey clip, both stages: 0.319 ms there, 0.284 ms here).
+template <int kP, bool kGuided, bool kWide, int kRows>
 __global__ __launch_bounds__(kMatchThreads) void match_kernel(
     StageDesc d, const float* __restrict__ source, const uint32_t* __restrict__ anchors,
     int anchor_count, int* __restrict__ counts, uint32_t* __restrict__ positions,
@@ -218,11 +220,10 @@ __global__ __launch_bounds__(kMatchThreads) void match_kernel(
     float* s_sel_dist = s_dyn + L.sel;
     int* s_sel_index = reinterpret_cast<int*>(s_sel_dist + selection_entries(d));
     int* s_sel_rank = s_sel_index + selection_entries(d);
-    float* s_ref = s_dyn + L.ref;
+    float* s_ref = reinterpret_cast<float*>(s_match4 + L.ref / 4);
 
     const int groups_x = (nx + 3) >> 2;
-    const bool paired = nt * ny * groups_x > kMatchThreads;
-    if (!paired) {
+    if (kRows == 1) {
         // Few candidates per thread and few wavefronts to cover a scalar
         // load's latency: the reference patch [c][t][y][x] in LDS.
         for (int i = threadIdx.x; i < match_channels * d.patch_dim; i += blockDim.x) {
@@ -237,8 +238,7 @@ __global__ __launch_bounds__(kMatchThreads) void match_kernel(
     constexpr int kRowLanes = 32;
     constexpr int kRowBatch = 8;
     const int row_lane = threadIdx.x % kRowLanes;
-    const auto scan = [&](auto rows_per, int ch) {
-        constexpr int kRows = decltype(rows_per)::value;
+    const auto scan = [&](int ch) {
         const int ny_items = (ny + kRows - 1) / kRows;
         const int items = nt * ny_items * groups_x;
         // The reference patch of this channel: uniform rows of the clip
@@ -285,50 +285,67 @@ __global__ __launch_bounds__(kMatchThreads) void match_kernel(
     };
     for (int ch = 0; ch < match_channels; ++ch) {
         __syncthreads();
-        for (int rx = row_lane; rx < rcols; rx += kRowLanes) {
-            int fr = 0;
-            int ry = threadIdx.x / kRowLanes;
-            // Batches of rows, their loads issued together.
-            while (fr < rframes) {
-                float value[kRowBatch];
-                int to[kRowBatch];
-#pragma unroll
-                for (int k = 0; k < kRowBatch; ++k) {
-                    while (ry >= rrows) {
-                        ry -= rrows;
-                        ++fr;
-                    }
-                    to[k] = -1;
-                    value[k] = 0.0F;
-                    if (fr < rframes) {
-                        int x0 = x_low;
-                        int y0 = y_low;
-                        int frame = t_low + fr;
-                        if (guided) {
-                            const int ti = fr / d.patch_time;
-                            x0 = s_frame_x_low[ti];
-                            y0 = s_frame_y_low[ti];
-                            frame = scheduled_frame(af, t_low, t_high, ti) + fr - ti * d.patch_time;
-                        }
-                        value[k] = video_at(source, d, x0 + rx, y0 + ry, frame, ch);
-                        to[k] = fr * plane + ry * pitch + rx;
-                    }
-                    ry += kMatchThreads / kRowLanes;
+        if (kRows == 1) {
+            // A sample per thread: few rows, fewer than a batch of them below.
+            const int region_plane = rrows * rcols;
+            for (int i = threadIdx.x; i < rframes * region_plane; i += kMatchThreads) {
+                const int fr = i / region_plane;
+                const int rem = i - fr * region_plane;
+                const int ry = rem / rcols;
+                const int rx = rem - ry * rcols;
+                int x0 = x_low;
+                int y0 = y_low;
+                int frame = t_low + fr;
+                if (guided) {
+                    const int ti = fr / d.patch_time;
+                    x0 = s_frame_x_low[ti];
+                    y0 = s_frame_y_low[ti];
+                    frame = scheduled_frame(af, t_low, t_high, ti) + fr - ti * d.patch_time;
                 }
+                s_region[fr * plane + ry * pitch + rx] = video_at(source, d, x0 + rx, y0 + ry, frame, ch);
+            }
+        } else {
+            for (int rx = row_lane; rx < rcols; rx += kRowLanes) {
+                int fr = 0;
+                int ry = threadIdx.x / kRowLanes;
+                // Batches of rows, their loads issued together.
+                while (fr < rframes) {
+                    float value[kRowBatch];
+                    int to[kRowBatch];
 #pragma unroll
-                for (int k = 0; k < kRowBatch; ++k) {
-                    if (to[k] >= 0) {
-                        s_region[to[k]] = value[k];
+                    for (int k = 0; k < kRowBatch; ++k) {
+                        while (ry >= rrows) {
+                            ry -= rrows;
+                            ++fr;
+                        }
+                        to[k] = -1;
+                        value[k] = 0.0F;
+                        if (fr < rframes) {
+                            int x0 = x_low;
+                            int y0 = y_low;
+                            int frame = t_low + fr;
+                            if (guided) {
+                                const int ti = fr / d.patch_time;
+                                x0 = s_frame_x_low[ti];
+                                y0 = s_frame_y_low[ti];
+                                frame = scheduled_frame(af, t_low, t_high, ti) + fr - ti * d.patch_time;
+                            }
+                            value[k] = video_at(source, d, x0 + rx, y0 + ry, frame, ch);
+                            to[k] = fr * plane + ry * pitch + rx;
+                        }
+                        ry += kMatchThreads / kRowLanes;
+                    }
+#pragma unroll
+                    for (int k = 0; k < kRowBatch; ++k) {
+                        if (to[k] >= 0) {
+                            s_region[to[k]] = value[k];
+                        }
                     }
                 }
             }
         }
         __syncthreads();
-        if (paired) {
-            scan(std::integral_constant<int, 2>{}, ch);
-        } else {
-            scan(std::integral_constant<int, 1>{}, ch);
-        }
+        scan(ch);
     }
     __syncthreads();
     select_and_write(d, s_dist, n, af, t_low, t_high, x_low, y_low, nx, per_frame, nt, s_hist,
@@ -725,23 +742,30 @@ hipError_t launch_match(const StageDesc& d, const float* source,
     const bool guided = offsets != nullptr;
     const bool wide = match_wide_rows(d, guided);
     const size_t shared = match_layout(d, d.patch, guided, wide).words * sizeof(float);
-#define VNLBHIP_MATCH(PV, GUIDED, WIDE)                                                          \
-    hipLaunchKernelGGL((match_kernel<PV, GUIDED, WIDE>), grid, block, shared, stream, d, source, \
-                       anchors, anchor_count, counts, positions, distances, offsets,             \
+    const bool paired = match_paired_rows(d);
+#define VNLBHIP_MATCH_ROWS(PV, GUIDED, WIDE, ROWS)                                                \
+    hipLaunchKernelGGL((match_kernel<PV, GUIDED, WIDE, ROWS>), grid, block, shared, stream, d,    \
+                       source, anchors, anchor_count, counts, positions, distances, offsets,      \
                        offsets_temporal)
+#define VNLBHIP_MATCH(PV, GUIDED, WIDE)                \
+    if (paired) {                                      \
+        VNLBHIP_MATCH_ROWS(PV, GUIDED, WIDE, 2);       \
+    } else {                                           \
+        VNLBHIP_MATCH_ROWS(PV, GUIDED, WIDE, 1);       \
+    }
     switch (d.patch) {
 #define VNLBHIP_MATCH_CASE(PV)                                       \
     case PV:                                                         \
         if (wide) {                                                  \
             if (guided) {                                            \
-                VNLBHIP_MATCH(PV, true, true);                       \
+                VNLBHIP_MATCH(PV, true, true)                        \
             } else {                                                 \
-                VNLBHIP_MATCH(PV, false, true);                      \
+                VNLBHIP_MATCH(PV, false, true)                       \
             }                                                        \
         } else if (guided) {                                         \
-            VNLBHIP_MATCH(PV, true, false);                          \
+            VNLBHIP_MATCH(PV, true, false)                           \
         } else if constexpr (narrow_unguided_patch(PV)) {            \
-            VNLBHIP_MATCH(PV, false, false);                         \
+            VNLBHIP_MATCH(PV, false, false)                          \
         } else {                                                     \
             return hipErrorInvalidValue;  /* past kMatchBudget */    \
         }                                                            \
@@ -764,6 +788,7 @@ hipError_t launch_match(const StageDesc& d, const float* source,
         VNLBHIP_MATCH_CASE(16)
 #undef VNLBHIP_MATCH_CASE
 #undef VNLBHIP_MATCH
+#undef VNLBHIP_MATCH_ROWS
     default:
         return hipErrorInvalidValue;
     }

@@ -54,7 +54,7 @@ __host__ __device__ inline int selection_entries(const StageDesc& d) {
 struct MatchLayout {
     int dist;   // candidate distances
     int sel;    // three selection arrays
-    int ref;    // the reference patch
+    int ref;    // the reference patch (16-byte aligned)
     int words;
 };
 
@@ -62,7 +62,7 @@ __host__ __device__ inline MatchLayout match_layout(const StageDesc& d, int patc
     MatchLayout L{};
     L.dist = match_region_floats(d.search_window, patch, d.search_bwd + d.search_fwd + 1, d.patch_time, guided, wide);
     L.sel = L.dist + window_candidates(d);
-    L.ref = L.sel + 3 * selection_entries(d);
+    L.ref = (L.sel + 3 * selection_entries(d) + 3) / 4 * 4;
     L.words = L.ref + d.dim;
     return L;
 }
@@ -74,6 +74,21 @@ __host__ __device__ inline MatchLayout match_layout(const StageDesc& d, int patc
 // from 138 patch frames on.
 __host__ __device__ inline bool match_wide_rows(const StageDesc& d, bool guided) {
     return match_layout(d, d.patch, guided, true).words * sizeof(float) <= kMatchLds;
+}
+
+// Whether a thread takes two candidate rows: where one row each (four
+// candidates) would fill the workgroup more than once.  Every anchor's window
+// is shifted inside the clip, so all have the same size.  Measured with one
+// and with two rows (8x8 patches of a 200x150 grey clip, matching of both
+// stages): 15x15x3 windows, 180 threads of one row, 0.350 and 0.387 ms;
+// 19x19x3, 285, 0.384 and 0.374 ms; 21x21x3, 378, 0.441 and 0.388 ms; 25x25x5,
+// 875, 1.109 and 0.991 ms.
+__host__ __device__ inline bool match_paired_rows(const StageDesc& d) {
+    const auto least = [](int a, int b) { return a < b ? a : b; };
+    const int nx = least(d.search_window, d.width - d.patch + 1);
+    const int ny = least(d.search_window, d.height - d.patch + 1);
+    const int nt = least(d.search_bwd + d.search_fwd + 1, d.total_frames - d.patch_time + 1);
+    return nt * ny * ((nx + 3) / 4) > kMatchThreads;
 }
 
 // Patches whose unguided stages within kMatchBudget may need narrow rows: the
