@@ -154,6 +154,11 @@ FilterLayout filter_layout(const StageDesc& d, int tile_words, bool alias) {
 // samples (more than a sample per team); else over the basis, which a group
 // of one round no longer needs once its rows are filtered (larger groups of
 // such a stage are added directly); none where the model leaves no room.
+// Groups of several rounds pay for the tile with a workgroup or two per compute
+// unit and gain all the same: Basic of a 640x360x6 clip, coupled YUV, rank 16,
+// 17 samples 6.6 ms without a tile, 5.4 with it, 24 samples 8.1 and 5.5, 40
+// samples 11.1 and 7.0; rank 4, 24 samples 8.0 and 2.9; one model per channel,
+// 24 samples 8.1 and 4.6; grey, 24 samples 4.1 and 2.0, 64 samples 6.8 and 3.7.
 constexpr size_t kFilterSharedLimit = 112 * 1024;
 FilterLayout filter_layout(const StageDesc& d) {
     const auto fits = [](const FilterLayout& L, size_t limit) {
