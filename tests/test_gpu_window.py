@@ -146,15 +146,21 @@ def test_reserve_then_no_allocation():
 
 
 def test_two_contexts_on_two_threads_match_one():
+    """Each thread's Final runs on the single context's Basic.  On its own, whose
+    samples differ by up to 6e-7 from run to run in the fast form (order of the
+    fp32 sums), Final may decide a near tie of two candidates otherwise, and
+    then one patch differs: chained, 41 to 226 of 300 runs in a row were
+    1.18e-4 from the first; on a fixed Basic all were within 6e-7."""
     noisy, _, bp, fp = workloads.make("yuv_pt2_tau200")
     x = _dev(noisy)
     want = {}
+    basic = {}
     one = vnlbhip.Context(0)
     try:
         for form in ("plain", "fast"):
             one.set_form(form)
-            b = one.stage(BASIC, bp, x)
-            want[form] = (b.cpu().numpy(), one.stage(FINAL, fp, x, b).cpu().numpy())
+            basic[form] = one.stage(BASIC, bp, x)
+            want[form] = (basic[form].cpu().numpy(), one.stage(FINAL, fp, x, basic[form]).cpu().numpy())
     finally:
         one.close()
     results = {}
@@ -169,7 +175,7 @@ def test_two_contexts_on_two_threads_match_one():
                 with torch.cuda.stream(stream):
                     for _ in range(3):
                         b = ctx.stage(BASIC, bp, x)
-                        f = ctx.stage(FINAL, fp, x, b)
+                        f = ctx.stage(FINAL, fp, x, basic[form])
                     stream.synchronize()
                     results[form] = (b.cpu().numpy(), f.cpu().numpy())
             finally:
